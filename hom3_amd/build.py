@@ -12,7 +12,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libhom3g.so")
 OBJDIR = os.path.join(HERE, "_build")
-SOURCES = ["abi.hip", "topology.hip", "stepper.hip", "brick.hip", "batch.hip", "adjoint.hip"]
+SOURCES = ["abi.hip", "topology.hip", "stepper.hip", "tile.hip", "brick.hip", "batch.hip", "adjoint.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("HOM3G_ARCH", "gfx950")
 

@@ -366,6 +366,7 @@ int hom3g_solver_build(hom3g_ctx* ctx, int sid) {
       S.kernel = HOM3G_KERNEL_GENERIC;
     }
     if (S.kernel != HOM3G_KERNEL_BRICK) S.brick_table = false;
+    solver_build_tiles(C, S);
     solver_alloc_state(C, S);
   });
 }

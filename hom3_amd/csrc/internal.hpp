@@ -166,6 +166,33 @@ struct StepGraph {
   ~StepGraph() { drop(); }
 };
 
+// zero-gradient Neumann: the ghost holds a copy of its boundary cell
+inline bool zero_gradient(const BCDesc& b) {
+  if (b.kind != HOM3G_BC_NEUMANN) return false;
+  for (int k = 0; k < b.nparams; ++k)
+    if (b.params[k] != 0.0) return false;
+  return true;
+}
+
+// Tiles (tile.hpp): runs of kTileCells consecutive cells with their face lists
+constexpr int kTileCells = 256;
+struct TileHdr {
+  int32_t halo0, ext0;  // the tile's first entries in halo_more and ext_more
+  int32_t inst;         // whose scalars (batches)
+  int32_t pad;
+  uint16_t n, nh;       // cells, halo cells
+  uint16_t ne[3];       // extra faces per direction
+  uint16_t first;       // first tile of its instance
+  double root, inv_root;  // cell length of level 0 and its reciprocal
+};
+struct TileTab {
+  DevBuf<TileHdr> hdr;
+  DevBuf<uint32_t> face, ext, ext_more;
+  DevBuf<uint8_t> lev;
+  DevBuf<int32_t> halo, halo_more;
+  long long ntile = 0;
+};
+
 struct SolverDev {
   int id = -1, grid_id = -1, solver_idx = 0;
   hom3g_physics P{};
@@ -215,6 +242,9 @@ struct SolverDev {
   bool dtmin_current = false;   // scal.dtmin holds the CFL minimum of the current lhs
   double h_uniform = 0;         // cell length of a uniform grid
   int kernel = HOM3G_KERNEL_GENERIC;
+  bool tile_ok = false;         // first-order Euler stages on tiles (tile.hpp)
+  bool tile_ghosts = false;     // some tile reads ghosts: filled before every stage
+  TileTab tile;
   StepGraph step_graph;
   // host-callback boundary conditions (staging of the ghosts they fill)
   bool has_host_bc = false, host_bc_ready = false;
@@ -285,6 +315,9 @@ int64_t grid_refine_region(Ctx& C, GridDev& G, int max_level, const hom3g_geomet
 int64_t grid_balance(Ctx& C, GridDev& G);
 void solver_build(Ctx& C, GridDev& G, SolverDev& S);
 void solver_build_partners(Ctx& C, SolverDev& S);
+
+// tile.hip: the solver's tiles when its stages can run on them
+void solver_build_tiles(Ctx& C, SolverDev& S);
 
 // stepper.hip
 void solver_alloc_state(Ctx& C, SolverDev& S);

@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "internal.hpp"
+#include "tile.hpp"
 
 namespace hom3g {
 
@@ -566,8 +567,8 @@ __global__ void __launch_bounds__(256) k_dt(const double* Q, long long ld, const
       for (int v = 0; v < ND + 2; ++v) q[v] = Q[v * ld + c];
       double cd;
       if (FAST) {
-        // the formula the brick kernels fuse into their last stage, so a
-        // brick solver's dt does not depend on where the minimum came from
+        // the formula the brick and tile kernels fuse into their last stage,
+        // so a solver's dt does not depend on where the minimum came from
         cd = cell_dt_fast<ND, PHYS == HOM3G_CNS>(q, h, pc);
       } else {
         const Prim<ND, double> w = primitives<ND>(q, pc.gamma, pc.gm1);
@@ -951,7 +952,7 @@ void launch_stage_fp32(Ctx& C, SolverDev& S, const void* in, bool in32, void* ou
 
 void launch_dt(Ctx& C, SolverDev& S) {
   const unsigned nb = nblk(S.n_int);
-  const bool fast = S.kernel == HOM3G_KERNEL_BRICK;
+  const bool fast = S.kernel == HOM3G_KERNEL_BRICK || S.tile_ok;
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, C.stream, (const double*)S.lhs.p, (long long)S.cap,
                        (const double*)S.length.p, (long long)S.n_int, S.pc, S.scal.p);
@@ -1407,12 +1408,58 @@ double solver_min_dt(Ctx& C, SolverDev& S) {
   return r;
 }
 
+// The stages of one step on tiles: the ghosts of a stage's input are filled
+// only where some tile reads them, the CFL bound of the new state and the
+// advance are fused into the last stage (10 launches a step before, 4 now).
+static void tile_steps(Ctx& C, SolverDev& S) {
+  const TileView t = tile_view(S.tile);
+  const unsigned grid = (unsigned)t.ntile;
+  const bool f32 = S.P.precision == HOM3G_FP32_STATE;
+  auto run = [&](const void* in, bool in32, void* out, bool out32, int kind, bool last) {
+    tile_stage(C, S.nd, t, S.pc, TileStage{in, S.lhs.p, out, in32, out32, (long long)S.cap, (long long)S.n_int, kind, last, last},
+               S.scal.p, grid);
+  };
+  auto ghosts = [&](bool stg) {
+    if (!S.tile_ghosts) return;
+    if (f32) solver_fill_ghosts(C, S, stg ? S.stg32.p : S.rhs32.p);
+    else solver_fill_ghosts(C, S, stg ? S.stg.p : S.rhs.p);
+  };
+  void* s1 = f32 ? (void*)S.rhs32.p : (void*)S.rhs.p;
+  void* s2 = f32 ? (void*)S.stg32.p : (void*)S.stg.p;
+  if (S.P.ti == HOM3G_TI_EULER_FWD) {
+    run(S.lhs.p, false, S.rhs.p, false, 0, true);
+    // lhs = rhs on the internal cells; the ghost slots keep this step's
+    // apply_bcs(lhs)
+    if (S.n_ghost) {
+      hipLaunchKernelGGL(k_copy_ghosts, dim3(nblk(S.n_ghost * S.nvars)), dim3(256), 0, C.stream,
+                         (const double*)S.lhs.p, S.rhs.p, (long long)S.cap, (long long)S.n_int,
+                         (long long)S.n_ghost, S.nvars);
+      H3_LAUNCH_CHECK();
+    }
+    std::swap(S.lhs.p, S.rhs.p);
+  } else if (S.P.ti == HOM3G_TI_HEUN_RK2) {
+    run(S.lhs.p, false, s1, f32, 4, false);
+    ghosts(false);
+    run(s1, f32, S.lhs.p, false, 1, true);
+  } else {
+    run(S.lhs.p, false, s1, f32, 0, false);
+    ghosts(false);
+    run(s1, f32, s2, f32, 2, false);
+    ghosts(true);
+    run(s2, f32, S.lhs.p, false, 3, true);
+  }
+  S.dtmin_current = true;
+}
+
 // one solve() (solver.hpp:140-145); skip_dt_reduction when force_dt was just
-// applied on the device for this step
-static void solve_one(Ctx& C, SolverDev& S, bool skip_dt_reduction) {
+// applied on the device for this step; last: the caller may read the lhs
+// ghosts after this step (they hold apply_bcs of the state the step began
+// with: tiles that read no ghost leave them to the last step of a solve)
+static void solve_one(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool last = true) {
   const bool brick = (S.kernel == HOM3G_KERNEL_BRICK);
-  if (!brick || S.brick_table) solver_fill_ghosts(C, S, S.lhs.p);
-  if (!skip_dt_reduction && !(brick && S.dtmin_current)) {
+  if (S.tile_ok ? (S.tile_ghosts || last || S.P.ti == HOM3G_TI_EULER_FWD) : (!brick || S.brick_table))
+    solver_fill_ghosts(C, S, S.lhs.p);
+  if (!skip_dt_reduction && !((brick || S.tile_ok) && S.dtmin_current)) {
     hipLaunchKernelGGL(k_reset_min, dim3(1), dim3(1), 0, C.stream, S.scal.p);
     launch_dt(C, S);
   }
@@ -1420,6 +1467,10 @@ static void solve_one(Ctx& C, SolverDev& S, bool skip_dt_reduction) {
   H3_LAUNCH_CHECK();
   S.dtmin_current = false;
   const double* src = S.source.p;
+  if (S.tile_ok) {
+    tile_steps(C, S);
+    return;
+  }
   if (brick) {
     // the next step's CFL minimum is fused into the last stage when the
     // boundary conditions leave the internal cells untouched
@@ -1544,7 +1595,7 @@ static uint64_t fnv_bytes(uint64_t h, const void* p, size_t n) {
 
 static uint64_t step_key(const SolverDev& S) {
   uint64_t h = 1469598103934665603ull;
-  const void* ptrs[] = {S.lhs.p, S.rhs.p, S.stg.p, S.rhs32.p, S.stg32.p, S.scal.p, S.source.p, S.nghbr.p};
+  const void* ptrs[] = {S.lhs.p, S.rhs.p, S.stg.p, S.rhs32.p, S.stg32.p, S.scal.p, S.source.p, S.nghbr.p, S.tile.hdr.p};
   h = fnv_bytes(h, ptrs, sizeof ptrs);
   const int64_t ints[] = {S.kernel, S.n_int, S.n_ghost, S.cap, S.uses_vortex_bc ? 1 : 0, S.dtmin_current ? 1 : 0};
   h = fnv_bytes(h, ints, sizeof ints);
@@ -1569,12 +1620,12 @@ static bool step_graph_ok(const Ctx& C, const SolverDev& S) {
 
 void solver_solve(Ctx& C, SolverDev& S, int nsteps) {
   if (nsteps < 3 || !step_graph_ok(C, S)) {
-    for (int i = 0; i < nsteps; ++i) solve_one(C, S, false);
+    for (int i = 0; i < nsteps; ++i) solve_one(C, S, false, i == nsteps - 1);
     return;
   }
   // one eager step brings the per-step flags to their steady values; the
   // same step is then captured once (capture does not run it) and replayed
-  solve_one(C, S, false);
+  solve_one(C, S, false, false);
   const bool dc = S.dtmin_current;
   const uint64_t key = step_key(S);
   StepGraph& G = S.step_graph;
@@ -1583,7 +1634,7 @@ void solver_solve(Ctx& C, SolverDev& S, int nsteps) {
     hipGraph_t g = nullptr;
     H3_HIP(hipStreamBeginCapture(C.stream, hipStreamCaptureModeThreadLocal));
     try {
-      solve_one(C, S, false);
+      solve_one(C, S, false, false);
     } catch (...) {
       (void)hipStreamEndCapture(C.stream, &g);
       if (g) (void)hipGraphDestroy(g);
@@ -1596,7 +1647,10 @@ void solver_solve(Ctx& C, SolverDev& S, int nsteps) {
     G.key = key;
     H3_REQUIRE(S.dtmin_current == dc, "a captured step must leave the step flags as it found them");
   }
-  for (int i = 1; i < nsteps; ++i) H3_HIP(hipGraphLaunch(G.exec, C.stream));
+  for (int i = 1; i < nsteps; ++i) {
+    if (i == nsteps - 1 && S.tile_ok && !S.tile_ghosts) solver_fill_ghosts(C, S, S.lhs.p);
+    H3_HIP(hipGraphLaunch(G.exec, C.stream));
+  }
 }
 
 // the CFL minimum of a solver's current lhs: the one a brick solver's last

@@ -1,0 +1,102 @@
+"""First-order Euler stages on tiles (tile.hip) where their face lists have
+edges: fewer cells than a tile, exactly one tile and one more, remainders,
+grids of several levels whose interface tiles overflow the halo and
+extra-face places, boundary conditions with and without ghosts, periodic
+images, and a masked domain with cut boundaries; each against the oracle."""
+import numpy as np
+import pytest
+
+import oracle as O
+from tests.scenarios import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+TI = {"euler_forward": O.TI_EULER_FWD, "runge_kutta_2": O.TI_HEUN_RK2, "ssp_rk3": O.TI_SSP_RK3}
+QUAD = [0.45, 0.55, 0.1, 0.2, 1.0, 1.0, -0.3, 0.1, 0.5, 0.4, 0.0, 0.0, 2.0, 1.5, 0.2, -0.2, 0.8, 0.9]
+BALL = [0.5, 0.5, 0.5, 0.3, 0.1, -0.2, 0.0, 1.0, 10.0, 0.0, 0.0, 0.1, 0.125, 0.1]
+
+
+def pair(nd, base, extra, radius, band, ti, bc, precision):
+    import hom3_amd as H
+    centre = [0.5, 0.4, 0.6][:nd]
+    ic = (O.IC_FOUR_QUADRANT, QUAD) if nd == 2 else (O.IC_SPHERE, BALL)
+    fixed = [0.1] * nd + [1.0, 2.5]
+    if bc == "dirichlet":
+        # the ghosts reflect the state at the fixed surface values, which only
+        # stays physical for states near them
+        ic = (O.IC_CONSTANT_PV, [0.1] * nd + [1.0, 0.4 * (2.5 - 0.5 * nd * 0.01)])
+    cond = {"neumann": (O.BC_EULER_NEUMANN, lambda: H.euler.bc.Neumann()),
+            "dirichlet": (O.BC_EULER_DIRICHLET, lambda: H.euler.bc.Dirichlet(fixed)),
+            "periodic": (O.BC_PERIODIC, lambda: H.Periodic())}[bc]
+    og = O.Grid(nd, [0.0] * nd, [1.0] * nd).min_level(base)
+    g = H.Grid(nd, [0.0] * nd, [1.0] * nd, base)
+    if extra:
+        og.refine_region(base + extra, O.geom(O.GEOM_SPHERE, centre, [radius]), band)
+        og.balance()
+        g.refine_region(base + extra, H.Sphere(centre, radius), band)
+        g.balance()
+    o = O.Solver(og, O.phys(physics=O.PHYS_EULER, nd=nd, ti=TI[ti], cfl=0.2))
+    prm = fixed if bc == "dirichlet" else []
+    for i, geo in enumerate(O.cube_boundaries(nd, [0.0] * nd, [1.0] * nd)):
+        o.append_bc(geo, cond[0], prm)
+    o.set_ic(*ic)
+    o.set_perturbation(5, 0.02)
+    o.initialize()
+    s = H.Solver(g, physics="euler", time_integration=ti, CFL=0.2, kernel="generic", precision=precision)
+    H.append_bcs(s, cond[1]())
+    s.set_initial_condition(*ic)
+    s.set_perturbation(5, 0.02)
+    s.initialize()
+    return o, s
+
+
+# (nd, base, extra, radius, band): 16 and 64 cells; one tile; ragged tiles of
+# refined grids; a ball refined twice (tiles over the level interfaces with
+# more than 384 halo cells and 128 extra faces a direction)
+GRIDS = [(2, 2, 0, 0, 0), (3, 2, 0, 0, 0), (2, 4, 0, 0, 0), (2, 4, 2, 0.2, 0.05), (3, 3, 1, 0.25, 0.1),
+         (3, 4, 2, 0.25, 0.02)]
+
+
+@pytest.mark.parametrize("bc", ["neumann", "dirichlet", "periodic"])
+@pytest.mark.parametrize("grid", GRIDS)
+def test_tiles_match_oracle(grid, bc):
+    if bc == "periodic" and grid[2]:
+        pytest.skip("periodic images are defined on uniform grids")
+    for ti in TI:
+        o, s = pair(*grid, ti, bc, "fp64")
+        assert s.kernel() == "generic" and s.first_gc == o.first_gc
+        o.solve(4)
+        s.solve(4)
+        n = o.first_gc
+        err = rel_l2(s.lhs[:, :n], o.get("lhs")[:, :n], grid[0])
+        assert np.max(err) <= 1e-12, (ti, err)
+        # the ghosts hold the boundary conditions of the last step's start
+        if n < s.ncells:
+            g = rel_l2(s.lhs[:, n:], o.get("lhs")[:, n:], grid[0])
+            assert np.max(g) <= 1e-12, (ti, g)
+        assert abs(s.time() - o.time()) <= 1e-13 * o.time()
+        s.close()
+
+
+def test_tiles_fp32_state():
+    o, s = pair(3, 4, 2, 0.25, 0.02, "ssp_rk3", "neumann", "fp32")
+    o.solve(4)
+    s.solve(4)
+    n = o.first_gc
+    err = rel_l2(s.lhs[:, :n], o.get("lhs")[:, :n], 3)
+    # FP32 rounding (6e-8) of two stage states and of the fluxes per step
+    assert 0 < np.max(err) <= 4 * 3 * 6e-8 * 8, err
+    s.close()
+
+
+def test_fused_dt_equals_the_reduction():
+    """The CFL bound fused into the last stage is the one a reduction over
+    the new state gives."""
+    _, s = pair(2, 4, 2, 0.2, 0.05, "ssp_rk3", "neumann", "fp64")
+    s.solve(5)
+    bound = s.min_dt()
+    s.solve(1)
+    assert s.dt() == bound
+    _, a = pair(2, 4, 2, 0.2, 0.05, "ssp_rk3", "neumann", "fp64")
+    a.solve(6)
+    np.testing.assert_array_equal(a.lhs, s.lhs)
