@@ -38,7 +38,7 @@ class Batch:
         return dict(block=b.value, tile=t.value, grid=g.value, items=n.value)
 
     def autotune(self):
-        """Pick block/tile/grid by timing stage 1; returns the choice and its time."""
+        """Pick the number of workgroups by timing stage 1; returns the launch shape and its time."""
         b, t, g, ms = C.c_int(), C.c_int(), C.c_int(), C.c_float()
         check(lib().hom3g_batch_autotune(self.ctx.h, self.id, C.byref(b), C.byref(t), C.byref(g), C.byref(ms)))
         return dict(block=b.value, tile=t.value, grid=g.value, stage_ms=ms.value)

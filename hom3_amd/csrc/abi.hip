@@ -867,7 +867,10 @@ int hom3g_batch_get_config(hom3g_ctx* ctx, int bid, int* block, int* tile, int* 
     if (block) *block = B.block;
     if (tile) *tile = B.tile;
     if (grid) *grid = B.grid;
-    if (nitems) *nitems = (int64_t)B.h_items.size();
+    if (nitems) {
+      *nitems = 0;
+      for (int64_t n : B.nint) *nitems += (n + B.tile - 1) / B.tile;
+    }
   });
 }
 

@@ -254,25 +254,16 @@ struct SolverDev {
   PinnedBuf<DevScalars> hbc_scal;
 };
 
-// Batched instances (batch.hip): concatenated internal cells, ghosts
-// resolved into the neighbour table, tiles of one instance as work items.
-struct BatchItem {
-  int inst, pad;
-  long long begin, end;
-};
-
+// Batched instances (batch.hip): each instance's internal cells from a
+// multiple of the tile size on, one list of tiles over all of them
 struct BatchDev {
   int nd = 0, nvars = 0, ninst = 0, precision = HOM3G_FP64, ti = HOM3G_TI_SSP_RK3;
   PhysConst pc{};
-  int64_t ncell = 0, nfine = 0;
-  DevBuf<double> U, S1d, S2d;   // nv x ncell, FP64 state and stage buffers
+  int64_t ncell = 0, ld = 0;    // cells of all instances; leading dimension of the state
+  DevBuf<double> U, S1d, S2d;   // nv x ld, FP64 state and stage buffers
   DevBuf<float> S1f, S2f;       // FP32 stage buffers
-  DevBuf<int32_t> nghbr;        // npos x ncell
-  DevBuf<int32_t> fine;         // 2^(nd-1) per face towards finer cells
-  DevBuf<double> len;           // ncell
+  TileTab tiles;
   DevBuf<DevScalars> scal;      // per instance
-  DevBuf<BatchItem> items;
-  std::vector<BatchItem> h_items;
   std::vector<int64_t> off, nint;
   int ncu = 256, block = 256, tile = 1024, grid = 1024;
   bool dtmin_current = false;

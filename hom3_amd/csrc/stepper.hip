@@ -1413,7 +1413,7 @@ double solver_min_dt(Ctx& C, SolverDev& S) {
 // advance are fused into the last stage (10 launches a step before, 4 now).
 static void tile_steps(Ctx& C, SolverDev& S) {
   const TileView t = tile_view(S.tile);
-  const unsigned grid = (unsigned)t.ntile;
+  const unsigned grid = tile_grid(t.ntile);
   const bool f32 = S.P.precision == HOM3G_FP32_STATE;
   auto run = [&](const void* in, bool in32, void* out, bool out32, int kind, bool last) {
     tile_stage(C, S.nd, t, S.pc, TileStage{in, S.lhs.p, out, in32, out32, (long long)S.cap, (long long)S.n_int, kind, last, last},

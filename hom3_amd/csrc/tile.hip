@@ -20,7 +20,7 @@
 // direction), in chunks of CE.
 //
 // Measured (one MI355X, refined blast, per step of three stages): 0.82 M
-// leaves FP64 0.258 -> 0.156 ms, 4.97 M leaves FP32 states 0.70 -> 0.49 ms
+// leaves FP64 0.258 -> 0.156 ms, 4.97 M leaves FP32 states 0.70 -> 0.45 ms
 // against the table-driven kernel and its separate ghost fills, CFL
 // reduction and advance.  A tile takes 7-9 us, most of it waiting: the chain
 // from the halo list to the halo states to the first face, and the two
@@ -29,6 +29,11 @@
 // a device copy's rate.  FP64 holds three workgroups per CU (LDS and 164
 // VGPRs), FP32 four (106 VGPRs; held to 96 or 80 it spills and runs 13% and
 // 60% slower).
+//
+// 2D batches (which evaluated every face from both sides too), per step:
+// 512 instances of 76.7 M cells FP64 7.05 -> 5.12 ms, FP32 states 5.59 ->
+// 4.14 ms; a pass of 40 steps of 12 instances (base grids 64^2 to 256^2, FP64)
+// 4.54 -> 3.78 ms.
 //
 // Boundaries.  A zero-gradient Neumann ghost holds a copy of its boundary
 // cell and a periodic one a copy of its image, so their faces read that cell

@@ -360,14 +360,14 @@ int hom3g_cht_misfit_adjoint(hom3g_ctx* ctx, int cns_sid, int heat_sid, double T
  * precision: HOM3G_FP64, or HOM3G_FP32_STATE (FP32 RK stage buffers and flux
  * arithmetic, FP64 U^n and RK accumulation). */
 int hom3g_batch_create(hom3g_ctx* ctx, const int* solver_ids, int n, int precision, int* batch_id);
-/* Launch shape: block threads (a multiple of 64, at most 512), tile = cells
- * per work item (at least block), grid = persistent workgroups.  Changing it
- * drops the captured graph. */
+/* Launch shape: grid = persistent workgroups.  block (a multiple of 64, at
+ * most 512) and tile (cells per work item, at least block) are checked and
+ * reported; the stages run on tiles of 256 cells with 256 threads whatever
+ * they are.  Changing it drops the captured graph. */
 int hom3g_batch_set_config(hom3g_ctx* ctx, int batch_id, int block, int tile, int grid);
 int hom3g_batch_get_config(hom3g_ctx* ctx, int batch_id, int* block, int* tile, int* grid, int64_t* nitems);
-/* Times stage 1 over block x tile x workgroups-per-CU candidates on the
- * current state (nothing is advanced) and keeps the fastest; outputs may be
- * NULL. */
+/* Times stage 1 over workgroups-per-CU candidates on the current state
+ * (nothing is advanced) and keeps the fastest; outputs may be NULL. */
 int hom3g_batch_autotune(hom3g_ctx* ctx, int batch_id, int* block, int* tile, int* grid, float* stage_ms);
 int hom3g_batch_solve(hom3g_ctx* ctx, int batch_id, int nsteps, int use_graph);
 /* nsteps steps between two events on the library stream; ms per step */
