@@ -34,6 +34,7 @@
 #include <functional>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 
 #include "brick_geo.hpp"
 #include "dual.hpp"
@@ -1899,13 +1900,17 @@ void csr(int64_t ntarget, size_t nent, Fill fill, std::vector<int32_t>& rp, std:
   for (size_t e = 0; e < nent; ++e) order[pos[tgt[e]]++] = (int32_t)e;
 }
 
-void build_rev_maps(Ctx& C, SolverDev& S, const SolverDev* other, RevMaps& M) {
+// (walks: with the slope-walk lists, which only the table-driven reverse
+// reads; most of the construction's time on 0.5 M cells)
+void build_rev_maps(Ctx& C, SolverDev& S, const SolverDev* other, bool walks, RevMaps& M) {
   const int64_t ld = S.cap, nc = S.n_int + S.n_ghost, ng = S.n_ghost;
   const int nd = S.nd;
-  std::vector<int32_t> nb((size_t)S.npos * ld), gb(ng), gim(ng), ghook(ng), gapp(ng), gpart(ng);
-  std::vector<double> len(ld);
-  S.nghbr.download(nb.data(), nb.size(), C.stream);
-  S.length.download(len.data(), ld, C.stream);
+  std::vector<int32_t> nb(walks ? (size_t)S.npos * ld : 0), gb(ng), gim(ng), ghook(ng), gapp(ng), gpart(ng);
+  std::vector<double> len(walks ? ld : 0);
+  if (walks) {
+    S.nghbr.download(nb.data(), nb.size(), C.stream);
+    S.length.download(len.data(), ld, C.stream);
+  }
   if (ng) {
     S.g_bndry.download(gb.data(), ng, C.stream);
     S.g_image.download(gim.data(), ng, C.stream);
@@ -1919,7 +1924,7 @@ void build_rev_maps(Ctx& C, SolverDev& S, const SolverDev* other, RevMaps& M) {
     return k == HOM3G_BC_ADIABATIC_NOSLIP || k == HOM3G_BC_ISOTHERMAL_NOSLIP || k == HOM3G_BC_CHT_FLUID;
   };
   std::vector<int32_t> rp, order;
-  if (S.P.physics == HOM3G_CNS) {
+  if (walks) {
     // the walk of slope (solver.hpp:596-623) for every cell and direction,
     // as slope_walk does it on the device
     struct E { int64_t tgt; int32_t src; uint8_t meta; double coef; };
@@ -2120,7 +2125,7 @@ struct RevWork {
   DevBuf<int4> urng;
   long long nu = 0;
   void alloc(Ctx& C, SolverDev& S, const SolverDev* other) {
-    build_rev_maps(C, S, other, maps);
+    build_rev_maps(C, S, other, S.P.physics == HOM3G_CNS && !tiled_rev(S), maps);
     const size_t ld = S.cap, nd = S.nd, nv = S.nvars;
     if (S.P.physics == HOM3G_HEAT) {
       // the heat reverse needs no work buffer
@@ -2179,6 +2184,20 @@ struct RevWork {
     H3_HIP(hipStreamSynchronize(C.stream));
   }
 };
+
+// S's reverse work, built at its first reverse sweep and kept with the
+// solver: the lists depend on its topology and conditions, which are fixed
+// when it is built, and on which solver it is coupled to
+RevWork& rev_work(Ctx& C, SolverDev& S, const SolverDev& other) {
+  if (!S.rev_work || S.rev_other != other.id) {
+    S.rev_work.reset();
+    auto w = std::make_shared<RevWork>();
+    w->alloc(C, S, &other);
+    S.rev_work = w;
+    S.rev_other = other.id;
+  }
+  return *static_cast<RevWork*>(S.rev_work.get());
+}
 
 // Ibar += adjoint of the stage's face fluxes (obar: adjoint of the stage
 // output, w: its weight)
@@ -2380,6 +2399,63 @@ __global__ void k_record_dt(const DevScalars* cs, const DevScalars* hs, double* 
 
 // ---- drivers -----------------------------------------------------------------
 
+// A call used to build the reverse lists on the host and allocate and free
+// each of its hundred or so buffers: 35 of the 45 ms of a gradient over 40
+// stored steps of the 64^3 channel, 62 of the 84 ms over 30 checkpointed
+// steps of the 128^3 one.  With the lists kept with the solver (rev_work),
+// the buffers from a kept workspace and the stages writing to them directly
+// they take 10.0 and 21.2 ms.
+//
+// The workspace of one adjoint call: the context's, or one of its own while
+// another thread's call holds that.  Waits for the call's work before giving
+// it back, also when an exception ends it.
+struct WsUse {
+  Ctx& C;
+  std::unique_lock<std::mutex> lock;
+  Workspace own;
+  explicit WsUse(Ctx& c) : C(c), lock(c.ws_lock, std::try_to_lock) {}
+  Workspace& get() { return lock.owns_lock() ? C.ws : own; }
+  ~WsUse() {
+    (void)hipStreamSynchronize(C.stream);
+    get().give_back();
+  }
+};
+template <class T>
+struct WsBuf {
+  T* p = nullptr;
+  size_t n = 0;
+  void alloc(Workspace& w, size_t count) {
+    p = static_cast<T*>(w.take(count * sizeof(T)));
+    n = count;
+  }
+  void download(T* h, size_t count, hipStream_t s) const {
+    H3_HIP(hipMemcpyAsync(h, p, count * sizeof(T), hipMemcpyDeviceToHost, s));
+  }
+};
+// a solver's stage buffers replaced for a while: the stages then write
+// straight to where the sweep keeps their states (SSP-RK3; forward Euler
+// exchanges its buffers itself)
+struct StageSwap {
+  SolverDev& S;
+  double *rhs = nullptr, *stg = nullptr;
+  bool on = false;
+  explicit StageSwap(SolverDev& s) : S(s) {}
+  void to(double* r, double* g) {
+    rhs = S.rhs.p;
+    stg = S.stg.p;
+    on = true;
+    S.rhs.p = r;
+    S.stg.p = g;
+  }
+  void back() {
+    if (!on) return;
+    S.rhs.p = rhs;
+    S.stg.p = stg;
+    on = false;
+  }
+  ~StageSwap() { back(); }
+};
+
 void cht_objective_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int nsteps, const double* dts,
                        double* dts_out, ChtRunStats& st, const double* obs) {
   check_pair(cns, heat);
@@ -2491,22 +2567,26 @@ void cht_adjoint_binomial(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, i
   const bool rk3 = cns.P.ti == HOM3G_TI_SSP_RK3;
   const long long nc = (long long)cns.nvars * cns.cap, nh = (long long)heat.nvars * heat.cap;
   const int nslot = std::min(slots, std::max(nsteps - 1, 1));
+  WsUse use(C);
+  Workspace& ws = use.get();
   {
     size_t free_b = 0, total_b = 0;
     H3_HIP(hipMemGetInfo(&free_b, &total_b));
+    free_b += ws.spare();
     const double need = (double)(nslot + 1 + (rk3 ? 3 : 1) + 10) * (double)(nc + nh) * sizeof(double);
     if (need > 0.9 * (double)free_b) throw Error(HOM3G_ERR_CAPACITY, "binomial checkpoints do not fit in device memory");
   }
   // stage buffers of the step being reversed
-  DevBuf<double> C0, C1, C2, H0, H1, H2;
-  C0.alloc(nc);
-  H0.alloc(nh);
-  if (rk3) { C1.alloc(nc); C2.alloc(nc); H1.alloc(nh); H2.alloc(nh); }
+  WsBuf<double> C0, C1, C2, H0, H1, H2;
+  C0.alloc(ws, nc);
+  H0.alloc(ws, nh);
+  if (rk3) { C1.alloc(ws, nc); C2.alloc(ws, nc); H1.alloc(ws, nh); H2.alloc(ws, nh); }
   // snapshot 0: the initial state; 1..nslot: the checkpoints
-  std::vector<DevBuf<double>> SC(nslot + 1), SH(nslot + 1);
-  for (int k = 0; k <= nslot; ++k) { SC[k].alloc(nc); SH[k].alloc(nh); }
-  DevBuf<DevScalars> SS;
-  SS.alloc(2 * (size_t)(nslot + 1));
+  std::vector<WsBuf<double>> SC(nslot + 1), SH(nslot + 1);
+  for (int k = 0; k <= nslot; ++k) { SC[k].alloc(ws, nc); SH[k].alloc(ws, nh); }
+  WsBuf<DevScalars> SS;
+  SS.alloc(ws, 2 * (size_t)(nslot + 1));
+  StageSwap keep_c(cns), keep_h(heat);
   auto save = [&](int k) {
     copyd(C, cns.lhs.p, SC[k].p, nc);
     copyd(C, heat.lhs.p, SH[k].p, nh);
@@ -2528,9 +2608,10 @@ void cht_adjoint_binomial(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, i
     solver_step(C, heat, true);
   };
   // forward sweep: J and the dts taken
-  DevBuf<double> dtrec, acc, term;
-  dtrec.alloc(2 * (size_t)std::max(nsteps, 1));
-  acc.alloc(1);
+  WsBuf<double> dtrec, acc;
+  DevBuf<double> term;
+  dtrec.alloc(ws, 2 * (size_t)std::max(nsteps, 1));
+  acc.alloc(ws, 1);
   zero(C, acc.p, 1);
   const Obs ob(C, heat, obs);
   save(0);
@@ -2550,9 +2631,9 @@ void cht_adjoint_binomial(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, i
   acc.download(&st.J, 1, C.stream);
   std::vector<double> dt_used(2 * (size_t)std::max(nsteps, 1));
   dtrec.download(dt_used.data(), dt_used.size(), C.stream);
-  DevBuf<double> finC, finH;
-  finC.alloc(nc);
-  finH.alloc(nh);
+  WsBuf<double> finC, finH;
+  finC.alloc(ws, nc);
+  finH.alloc(ws, nh);
   copyd(C, cns.lhs.p, finC.p, nc);
   copyd(C, heat.lhs.p, finH.p, nh);
   DevScalars fsc, fsh;
@@ -2561,13 +2642,11 @@ void cht_adjoint_binomial(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, i
   H3_HIP(hipStreamSynchronize(C.stream));
 
   // reverse sweep
-  RevWork Wc, Wh;
-  Wc.alloc(C, cns, &heat);
-  Wh.alloc(C, heat, &cns);
-  DevBuf<double> Cn1, Cn, Hn1, Hn, Ic, Oc, Ih, Oh, Sbar, Cend, Hend, OS;
-  for (DevBuf<double>* b : {&Cn1, &Cn, &Ic, &Oc, &Cend}) b->alloc(nc);
-  for (DevBuf<double>* b : {&Hn1, &Hn, &Ih, &Oh, &Sbar, &Hend}) b->alloc(nh);
-  OS.alloc(std::max<size_t>(1, (size_t)(heat.nd + 3) * heat.n_ghost));
+  RevWork &Wc = rev_work(C, cns, heat), &Wh = rev_work(C, heat, cns);
+  WsBuf<double> Cn1, Cn, Hn1, Hn, Ic, Oc, Ih, Oh, Sbar, Cend, Hend, OS;
+  for (WsBuf<double>* b : {&Cn1, &Cn, &Ic, &Oc, &Cend}) b->alloc(ws, nc);
+  for (WsBuf<double>* b : {&Hn1, &Hn, &Ih, &Oh, &Sbar, &Hend}) b->alloc(ws, nh);
+  OS.alloc(ws, std::max<size_t>(1, (size_t)(heat.nd + 3) * heat.n_ghost));
   zero(C, Cn1.p, nc);
   zero(C, Hn1.p, nh);
   zero(C, Sbar.p, nh);
@@ -2590,12 +2669,13 @@ void cht_adjoint_binomial(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, i
     cns.dtmin_current = heat.dtmin_current = false;
     solver_fill_ghosts(C, cns, cns.lhs.p);
     copyd(C, cns.lhs.p, C0.p, nc);
-    solver_step(C, cns, true);
-    if (rk3) { copyd(C, cns.rhs.p, C1.p, nc); copyd(C, cns.stg.p, C2.p, nc); }
+    if (rk3) { keep_c.to(C1.p, C2.p); keep_h.to(H1.p, H2.p); }
+    solver_step(C, cns, true, true);
     solver_fill_ghosts(C, heat, heat.lhs.p);
     copyd(C, heat.lhs.p, H0.p, nh);
-    solver_step(C, heat, true);
-    if (rk3) { copyd(C, heat.rhs.p, H1.p, nh); copyd(C, heat.stg.p, H2.p, nh); }
+    solver_step(C, heat, true, true);
+    keep_c.back();
+    keep_h.back();
     copyd(C, cns.lhs.p, Cend.p, nc);
     copyd(C, heat.lhs.p, Hend.p, nh);
     const double dtc = dt_used[2 * n], dth = dt_used[2 * n + 1];
@@ -2679,9 +2759,12 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
   const int K = store_all ? std::max(nsteps, 1) : ckpt_every, nseg = (nsteps + K - 1) / K;
   const int KS = std::min(K, nsteps);
   const int per_step = rk3 ? 3 : 1;
+  WsUse use(C);
+  Workspace& ws = use.get();
   if (store_all) {
     size_t free_b = 0, total_b = 0;
     H3_HIP(hipMemGetInfo(&free_b, &total_b));
+    free_b += ws.spare();
     const double need = (double)KS * per_step * (double)(nc + nh) * sizeof(double);
     if (need > 0.9 * (double)free_b) {
       char msg[256];
@@ -2690,29 +2773,30 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
       throw Error(HOM3G_ERR_CAPACITY, msg);
     }
   }
-  std::vector<DevBuf<double>> C0(KS), C1(rk3 ? KS : 0), C2(rk3 ? KS : 0), H0(KS), H1(rk3 ? KS : 0), H2(rk3 ? KS : 0);
+  std::vector<WsBuf<double>> C0(KS), C1(rk3 ? KS : 0), C2(rk3 ? KS : 0), H0(KS), H1(rk3 ? KS : 0), H2(rk3 ? KS : 0);
   for (int j = 0; j < KS; ++j) {
-    C0[j].alloc(nc);
-    H0[j].alloc(nh);
-    if (rk3) { C1[j].alloc(nc); C2[j].alloc(nc); H1[j].alloc(nh); H2[j].alloc(nh); }
+    C0[j].alloc(ws, nc);
+    H0[j].alloc(ws, nh);
+    if (rk3) { C1[j].alloc(ws, nc); C2[j].alloc(ws, nc); H1[j].alloc(ws, nh); H2[j].alloc(ws, nh); }
   }
   // the dts both solvers took (set_dt clamps the forced dt at the end time)
-  DevBuf<double> dtrec;
-  dtrec.alloc(2 * (size_t)std::max(nsteps, 1));
+  WsBuf<double> dtrec;
+  dtrec.alloc(ws, 2 * (size_t)std::max(nsteps, 1));
+  StageSwap keep_c(cns), keep_h(heat);
   // one coupled step that keeps the stage inputs of both solvers in slot j
-  // (the ghost fills are those solver_step performs; repeating them changes
-  // nothing)
+  // (the stages write theirs straight to the slot)
   auto record_step = [&](int n, int j) {
     hipLaunchKernelGGL(k_force_pair, dim3(1), dim3(1), 0, C.stream, cns.scal.p, heat.scal.p, dts[n], scaling);
     H3_LAUNCH_CHECK();
     solver_fill_ghosts(C, cns, cns.lhs.p);
     copyd(C, cns.lhs.p, C0[j].p, nc);
-    solver_step(C, cns, true);
-    if (rk3) { copyd(C, cns.rhs.p, C1[j].p, nc); copyd(C, cns.stg.p, C2[j].p, nc); }
+    if (rk3) { keep_c.to(C1[j].p, C2[j].p); keep_h.to(H1[j].p, H2[j].p); }
+    solver_step(C, cns, true, true);
     solver_fill_ghosts(C, heat, heat.lhs.p);
     copyd(C, heat.lhs.p, H0[j].p, nh);
-    solver_step(C, heat, true);
-    if (rk3) { copyd(C, heat.rhs.p, H1[j].p, nh); copyd(C, heat.stg.p, H2[j].p, nh); }
+    solver_step(C, heat, true, true);
+    keep_c.back();
+    keep_h.back();
   };
 
   // forward sweep: checkpoints (state and scalars) every K steps (in device
@@ -2722,15 +2806,17 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
   if (!store_all) {
     size_t free_b = 0, total_b = 0;
     H3_HIP(hipMemGetInfo(&free_b, &total_b));
+    free_b += ws.spare();
     const double need = (double)nseg * (double)(nc + nh) * sizeof(double);
     host_ck = C.ckpt_memory == HOM3G_CKPT_HOST || (C.ckpt_memory == HOM3G_CKPT_AUTO && need > 0.8 * (double)free_b);
   }
-  std::vector<DevBuf<double>> ckC(store_all || host_ck ? 0 : nseg), ckH(store_all || host_ck ? 0 : nseg);
+  std::vector<WsBuf<double>> ckC(store_all || host_ck ? 0 : nseg), ckH(store_all || host_ck ? 0 : nseg);
   std::vector<PinnedBuf<double>> hkC(host_ck ? nseg : 0), hkH(host_ck ? nseg : 0);
-  DevBuf<DevScalars> ckS;
-  ckS.alloc(2 * (size_t)std::max(nseg, 1));
-  DevBuf<double> acc, term;
-  acc.alloc(1);
+  WsBuf<DevScalars> ckS;
+  ckS.alloc(ws, 2 * (size_t)std::max(nseg, 1));
+  WsBuf<double> acc;
+  DevBuf<double> term;
+  acc.alloc(ws, 1);
   zero(C, acc.p, 1);
   const Obs ob(C, heat, obs);
   H3_HIP(hipEventRecord(C.ev0, C.stream));
@@ -2748,8 +2834,8 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
           H3_HIP(hipMemcpyAsync(hkC[n / K].p, cns.lhs.p, nc * sizeof(double), hipMemcpyDeviceToHost, C.stream));
           H3_HIP(hipMemcpyAsync(hkH[n / K].p, heat.lhs.p, nh * sizeof(double), hipMemcpyDeviceToHost, C.stream));
         } else {
-          ckC[n / K].alloc(nc);
-          ckH[n / K].alloc(nh);
+          ckC[n / K].alloc(ws, nc);
+          ckH[n / K].alloc(ws, nh);
           copyd(C, cns.lhs.p, ckC[n / K].p, nc);
           copyd(C, heat.lhs.p, ckH[n / K].p, nh);
         }
@@ -2773,9 +2859,9 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
   std::vector<double> dt_used(2 * (size_t)std::max(nsteps, 1));
   dtrec.download(dt_used.data(), dt_used.size(), C.stream);
   // the solvers end at step N; keep their final state and scalars
-  DevBuf<double> finC, finH;
-  finC.alloc(nc);
-  finH.alloc(nh);
+  WsBuf<double> finC, finH;
+  finC.alloc(ws, nc);
+  finH.alloc(ws, nh);
   copyd(C, cns.lhs.p, finC.p, nc);
   copyd(C, heat.lhs.p, finH.p, nh);
   DevScalars fsc, fsh;
@@ -2784,16 +2870,14 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
   H3_HIP(hipStreamSynchronize(C.stream));
 
   // reverse sweep
-  RevWork Wc, Wh;
-  Wc.alloc(C, cns, &heat);
-  Wh.alloc(C, heat, &cns);
-  DevBuf<double> Cn1, Cn, Hn1, Hn, Ic, Oc, Ih, Oh, Sbar, Cend, Hend, OS;
-  for (DevBuf<double>* b : {&Cn1, &Cn, &Ic, &Oc}) b->alloc(nc);
-  for (DevBuf<double>* b : {&Hn1, &Hn, &Ih, &Oh, &Sbar}) b->alloc(nh);
-  OS.alloc(std::max<size_t>(1, (size_t)(heat.nd + 3) * heat.n_ghost));
+  RevWork &Wc = rev_work(C, cns, heat), &Wh = rev_work(C, heat, cns);
+  WsBuf<double> Cn1, Cn, Hn1, Hn, Ic, Oc, Ih, Oh, Sbar, Cend, Hend, OS;
+  for (WsBuf<double>* b : {&Cn1, &Cn, &Ic, &Oc}) b->alloc(ws, nc);
+  for (WsBuf<double>* b : {&Hn1, &Hn, &Ih, &Oh, &Sbar}) b->alloc(ws, nh);
+  OS.alloc(ws, std::max<size_t>(1, (size_t)(heat.nd + 3) * heat.n_ghost));
   if (!store_all) {
-    Cend.alloc(nc);
-    Hend.alloc(nh);
+    Cend.alloc(ws, nc);
+    Hend.alloc(ws, nh);
   }
   const double* CendP = store_all ? finC.p : Cend.p;
   const double* HendP = store_all ? finH.p : Hend.p;

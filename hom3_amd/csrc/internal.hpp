@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -245,6 +246,8 @@ struct SolverDev {
   bool tile_ok = false;         // first-order Euler stages on tiles (tile.hpp)
   bool tile_ghosts = false;     // some tile reads ghosts: filled before every stage
   TileTab tile;
+  std::shared_ptr<void> rev_work;  // index lists and work buffers of the reverse sweep (adjoint.hip)
+  int rev_other = -1;              // the coupled solver they were built with
   StepGraph step_graph;
   // host-callback boundary conditions (staging of the ghosts they fill)
   bool has_host_bc = false, host_bc_ready = false;
@@ -271,7 +274,68 @@ struct BatchDev {
   hipGraphExec_t exec = nullptr;
 };
 
+// Device workspace handed out in pieces and kept between calls: the adjoint
+// takes some hundred buffers per call, and allocating and freeing each cost
+// more than the sweeps.  What exceeds kKeep is given back at the end of a
+// call, the rest with its owner.
+struct Workspace {
+  static constexpr size_t kChunk = size_t(64) << 20, kKeep = size_t(2) << 30;
+  struct Chunk {
+    DevBuf<char> buf;
+    size_t used = 0;
+  };
+  std::vector<std::unique_ptr<Chunk>> chunks;
+  void* take(size_t bytes) {
+    bytes = (bytes + 255) & ~size_t(255);
+    for (auto& c : chunks)
+      if (c->buf.n - c->used >= bytes) {
+        void* p = c->buf.p + c->used;
+        c->used += bytes;
+        return p;
+      }
+    auto c = std::make_unique<Chunk>();
+    const size_t want = bytes > kChunk ? bytes : kChunk;
+    try {
+      c->buf.alloc(want);
+    } catch (const Error&) {
+      // short of memory: what lies unused goes first
+      (void)hipGetLastError();
+      drop_unused();
+      c->buf.alloc(want);
+    }
+    c->used = bytes;
+    chunks.push_back(std::move(c));
+    return chunks.back()->buf.p;
+  }
+  void drop_unused() {
+    for (size_t k = 0; k < chunks.size();)
+      if (chunks[k]->used == 0) chunks.erase(chunks.begin() + k);
+      else ++k;
+  }
+  // bytes kept and not handed out
+  size_t spare() const {
+    size_t n = 0;
+    for (auto& c : chunks) n += c->buf.n - c->used;
+    return n;
+  }
+  // end of a call: nothing handed out is in use any more
+  void give_back() {
+    size_t total = 0;
+    for (size_t k = 0; k < chunks.size();) {
+      chunks[k]->used = 0;
+      if (total + chunks[k]->buf.n > kKeep) {
+        chunks.erase(chunks.begin() + k);
+      } else {
+        total += chunks[k]->buf.n;
+        ++k;
+      }
+    }
+  }
+};
+
 struct Ctx {
+  Workspace ws;             // of the adjoint sweep that holds ws_lock
+  std::mutex ws_lock;
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -316,7 +380,8 @@ void solver_impose_ic(Ctx& C, SolverDev& S, int kind, const double* params, int 
 void solver_init_time(Ctx& C, SolverDev& S);
 void solver_solve(Ctx& C, SolverDev& S, int nsteps);
 // one step (solver.hpp:140-145); skip_dt_reduction when the dt is forced
-void solver_step(Ctx& C, SolverDev& S, bool skip_dt_reduction);
+// (lhs_ghosts: the ghosts of lhs are already those of its current state)
+void solver_step(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool lhs_ghosts = false);
 void solver_min_dt_device(Ctx& C, SolverDev& S, unsigned long long* out_dev);
 double solver_min_dt(Ctx& C, SolverDev& S);
 void solver_conservation_sums(Ctx& C, SolverDev& S, double* out);

@@ -1455,9 +1455,11 @@ static void tile_steps(Ctx& C, SolverDev& S) {
 // applied on the device for this step; last: the caller may read the lhs
 // ghosts after this step (they hold apply_bcs of the state the step began
 // with: tiles that read no ghost leave them to the last step of a solve)
-static void solve_one(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool last = true) {
+static void solve_one(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool last = true, bool lhs_ghosts = false) {
   const bool brick = (S.kernel == HOM3G_KERNEL_BRICK);
-  if (S.tile_ok ? (S.tile_ghosts || last || S.P.ti == HOM3G_TI_EULER_FWD) : (!brick || S.brick_table))
+  if (lhs_ghosts) {
+    // filled by the caller
+  } else if (S.tile_ok ? (S.tile_ghosts || last || S.P.ti == HOM3G_TI_EULER_FWD) : (!brick || S.brick_table))
     solver_fill_ghosts(C, S, S.lhs.p);
   if (!skip_dt_reduction && !((brick || S.tile_ok) && S.dtmin_current)) {
     hipLaunchKernelGGL(k_reset_min, dim3(1), dim3(1), 0, C.stream, S.scal.p);
@@ -1584,7 +1586,9 @@ static void solve_one(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool last = 
   }
 }
 
-void solver_step(Ctx& C, SolverDev& S, bool skip_dt_reduction) { solve_one(C, S, skip_dt_reduction); }
+void solver_step(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool lhs_ghosts) {
+  solve_one(C, S, skip_dt_reduction, true, lhs_ghosts);
+}
 
 // FNV-1a over the bytes a captured step depends on
 static uint64_t fnv_bytes(uint64_t h, const void* p, size_t n) {
