@@ -2388,12 +2388,9 @@ void rev_solver(Ctx& C, SolverDev& S, const AdjTopo& t, RevWork& W, const RevArg
   }
 }
 
-// the dt each solver took in the step just run (set_dt may clamp the forced
-// dt at the end time), kept for the reverse sweep
-__global__ void k_record_dt(const DevScalars* cs, const DevScalars* hs, double* out) {
-  out[0] = cs->dt;
-  out[1] = hs->dt;
-}
+// steps whose dt force_pair_dt has set, without and with lhs ghosts in place
+const StepFlags kForced = [] { StepFlags f; f.skip_dt_reduction = f.dt_set = true; return f; }();
+const StepFlags kForcedFilled = [] { StepFlags f = kForced; f.lhs_ghosts = true; return f; }();
 
 }  // namespace
 
@@ -2469,11 +2466,9 @@ void cht_objective_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int 
   H3_HIP(hipEventRecord(C.ev0, C.stream));
   for (int n = 0; n < nsteps; ++n) {
     if (dts) {
-      hipLaunchKernelGGL(k_force_pair, dim3(1), dim3(1), 0, C.stream, cns.scal.p, heat.scal.p, dts[n], scaling);
-      H3_LAUNCH_CHECK();
-      cns.dtmin_current = heat.dtmin_current = false;
-      solver_step(C, cns, true);
-      solver_step(C, heat, true);
+      force_pair_dt(C, cns, heat, dts[n], scaling, nullptr);
+      solver_step(C, cns, kForced);
+      solver_step(C, heat, kForced);
     } else {
       couple_cht_step(C, cns, heat, Tr0);
     }
@@ -2600,12 +2595,10 @@ void cht_adjoint_binomial(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, i
     H3_HIP(hipMemcpyAsync(heat.scal.p, SS.p + 2 * k + 1, sizeof(DevScalars), hipMemcpyDeviceToDevice, C.stream));
     cns.dtmin_current = heat.dtmin_current = false;
   };
-  auto advance = [&](int n) {
-    hipLaunchKernelGGL(k_force_pair, dim3(1), dim3(1), 0, C.stream, cns.scal.p, heat.scal.p, dts[n], scaling);
-    H3_LAUNCH_CHECK();
-    cns.dtmin_current = heat.dtmin_current = false;
-    solver_step(C, cns, true);
-    solver_step(C, heat, true);
+  auto advance = [&](int n, double* rec = nullptr) {
+    force_pair_dt(C, cns, heat, dts[n], scaling, rec);
+    solver_step(C, cns, kForced);
+    solver_step(C, heat, kForced);
   };
   // forward sweep: J and the dts taken
   WsBuf<double> dtrec, acc;
@@ -2617,10 +2610,7 @@ void cht_adjoint_binomial(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, i
   save(0);
   H3_HIP(hipEventRecord(C.ev0, C.stream));
   for (int n = 0; n < nsteps; ++n) {
-    advance(n);
-    hipLaunchKernelGGL(k_record_dt, dim3(1), dim3(1), 0, C.stream, (const DevScalars*)cns.scal.p,
-                       (const DevScalars*)heat.scal.p, dtrec.p + 2 * n);
-    H3_LAUNCH_CHECK();
+    advance(n, dtrec.p + 2 * n);
     if (!ob.p) objective_launch(C, heat, cns, th, nullptr, nullptr, term, acc.p);
   }
   if (ob.p) misfit_launch(C, heat, ob.p, nullptr, term, acc.p);
@@ -2664,16 +2654,14 @@ void cht_adjoint_binomial(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, i
   // step n from the state at n held by the solvers: record its stage inputs,
   // keep the state at n + 1, reverse it
   auto reverse_one = [&](int n) {
-    hipLaunchKernelGGL(k_force_pair, dim3(1), dim3(1), 0, C.stream, cns.scal.p, heat.scal.p, dts[n], scaling);
-    H3_LAUNCH_CHECK();
-    cns.dtmin_current = heat.dtmin_current = false;
+    force_pair_dt(C, cns, heat, dts[n], scaling, nullptr);
     solver_fill_ghosts(C, cns, cns.lhs.p);
     copyd(C, cns.lhs.p, C0.p, nc);
     if (rk3) { keep_c.to(C1.p, C2.p); keep_h.to(H1.p, H2.p); }
-    solver_step(C, cns, true, true);
+    solver_step(C, cns, kForcedFilled);
     solver_fill_ghosts(C, heat, heat.lhs.p);
     copyd(C, heat.lhs.p, H0.p, nh);
-    solver_step(C, heat, true, true);
+    solver_step(C, heat, kForcedFilled);
     keep_c.back();
     keep_h.back();
     copyd(C, cns.lhs.p, Cend.p, nc);
@@ -2785,16 +2773,15 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
   StageSwap keep_c(cns), keep_h(heat);
   // one coupled step that keeps the stage inputs of both solvers in slot j
   // (the stages write theirs straight to the slot)
-  auto record_step = [&](int n, int j) {
-    hipLaunchKernelGGL(k_force_pair, dim3(1), dim3(1), 0, C.stream, cns.scal.p, heat.scal.p, dts[n], scaling);
-    H3_LAUNCH_CHECK();
+  auto record_step = [&](int n, int j, double* rec) {
+    force_pair_dt(C, cns, heat, dts[n], scaling, rec);
     solver_fill_ghosts(C, cns, cns.lhs.p);
     copyd(C, cns.lhs.p, C0[j].p, nc);
     if (rk3) { keep_c.to(C1[j].p, C2[j].p); keep_h.to(H1[j].p, H2[j].p); }
-    solver_step(C, cns, true, true);
+    solver_step(C, cns, kForcedFilled);
     solver_fill_ghosts(C, heat, heat.lhs.p);
     copyd(C, heat.lhs.p, H0[j].p, nh);
-    solver_step(C, heat, true, true);
+    solver_step(C, heat, kForcedFilled);
     keep_c.back();
     keep_h.back();
   };
@@ -2822,7 +2809,7 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
   H3_HIP(hipEventRecord(C.ev0, C.stream));
   for (int n = 0; n < nsteps; ++n) {
     if (store_all) {
-      record_step(n, n);
+      record_step(n, n, dtrec.p + 2 * n);
     } else {
       if (n % K == 0) {
         H3_HIP(hipMemcpyAsync(ckS.p + 2 * (n / K), cns.scal.p, sizeof(DevScalars), hipMemcpyDeviceToDevice, C.stream));
@@ -2840,14 +2827,10 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
           copyd(C, heat.lhs.p, ckH[n / K].p, nh);
         }
       }
-      hipLaunchKernelGGL(k_force_pair, dim3(1), dim3(1), 0, C.stream, cns.scal.p, heat.scal.p, dts[n], scaling);
-      H3_LAUNCH_CHECK();
-      solver_step(C, cns, true);
-      solver_step(C, heat, true);
+      force_pair_dt(C, cns, heat, dts[n], scaling, dtrec.p + 2 * n);
+      solver_step(C, cns, kForced);
+      solver_step(C, heat, kForced);
     }
-    hipLaunchKernelGGL(k_record_dt, dim3(1), dim3(1), 0, C.stream, (const DevScalars*)cns.scal.p,
-                       (const DevScalars*)heat.scal.p, dtrec.p + 2 * n);
-    H3_LAUNCH_CHECK();
     if (!ob.p) objective_launch(C, heat, cns, th, nullptr, nullptr, term, acc.p);
   }
   if (ob.p) misfit_launch(C, heat, ob.p, nullptr, term, acc.p);
@@ -2909,7 +2892,7 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
         copyd(C, ckC[sg].p, cns.lhs.p, nc);
         copyd(C, ckH[sg].p, heat.lhs.p, nh);
       }
-      for (int j = 0; j < len; ++j) record_step(n0 + j, j);
+      for (int j = 0; j < len; ++j) record_step(n0 + j, j, nullptr);
       copyd(C, cns.lhs.p, Cend.p, nc);
       copyd(C, heat.lhs.p, Hend.p, nh);
     }

@@ -379,9 +379,20 @@ void solver_alloc_state(Ctx& C, SolverDev& S);
 void solver_impose_ic(Ctx& C, SolverDev& S, int kind, const double* params, int np);
 void solver_init_time(Ctx& C, SolverDev& S);
 void solver_solve(Ctx& C, SolverDev& S, int nsteps);
-// one step (solver.hpp:140-145); skip_dt_reduction when the dt is forced
-// (lhs_ghosts: the ghosts of lhs are already those of its current state)
-void solver_step(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool lhs_ghosts = false);
+// one step (solver.hpp:140-145)
+struct StepFlags {
+  bool skip_dt_reduction = false;  // the dt is forced for this step
+  bool dt_set = false;             // set_dt is done (couple_cht_step, force_pair_dt)
+  bool lhs_ghosts = false;         // the ghosts of lhs are those of its current state
+  // the caller may read the lhs ghosts after this step (they hold apply_bcs of
+  // the state the step began with: tiles that read no ghost leave them to the
+  // last step of a solve)
+  bool last = true;
+};
+void solver_step(Ctx& C, SolverDev& S, const StepFlags& f);
+// a prescribed dt for the coupled pair's next step, set (StepFlags::dt_set);
+// rec: device memory for the two dts taken, or null
+void force_pair_dt(Ctx& C, SolverDev& cns, SolverDev& heat, double dt, double scaling, double* rec);
 void solver_min_dt_device(Ctx& C, SolverDev& S, unsigned long long* out_dev);
 double solver_min_dt(Ctx& C, SolverDev& S);
 void solver_conservation_sums(Ctx& C, SolverDev& S, double* out);

@@ -163,9 +163,8 @@ struct StageArgsT {
   const TIn* in;
   const double* base;
   TOut* out;
-  const double* src;  // per-cell volumetric source (heat) or null
-  int kind;           // 0: (in+nf)+src  1: 0.5*((base+in)+nf)  2: 0.75*base+0.25*((in+nf)+src)
-                      // 3: (1/3)*base+(2/3)*((in+nf)+src)  4: in+nf
+  int kind;           // 0, 4: in+nf  1: 0.5*((base+in)+nf)  2: 0.75*base+0.25*(in+nf)
+                      // 3: (1/3)*base+(2/3)*(in+nf)
 };
 using StageArgs = StageArgsT<double, double>;
 
@@ -237,8 +236,7 @@ __device__ __forceinline__ long long xcd_block() {
 template <int ND, int PHYS, class TIn, class TOut>
 __global__ void __launch_bounds__(256) k_stage_generic(GenTopo t, HookTable H, PhysConst pc, StageArgsT<TIn, TOut> a,
                                                        const DevScalars* scal) {
-  static_assert(PHYS != HOM3G_HEAT || (sizeof(TIn) == 8 && sizeof(TOut) == 8),
-                "FP32 heat stages run k_heat_stage32");
+  static_assert(PHYS != HOM3G_HEAT, "heat stages run k_heat_stage");
   // the boundary-hook kinds in LDS: indexed per lane (a dynamically indexed
   // kernel argument would be copied to scratch memory by every thread)
   __shared__ int hk[kMaxBC];
@@ -253,7 +251,7 @@ __global__ void __launch_bounds__(256) k_stage_generic(GenTopo t, HookTable H, P
   const long long blk = (PHYS == HOM3G_CNS) ? xcd_block() : (long long)blockIdx.x;
   const long long c = blk * blockDim.x + threadIdx.x;
   if (c >= t.n_int) return;
-  constexpr int NV = (PHYS == HOM3G_HEAT) ? 1 : ND + 2;
+  constexpr int NV = ND + 2;
   // the flux arithmetic: FP64, or FP32 with FP32 stage states (the RK
   // combination below stays FP64)
   using TC = std::conditional_t<sizeof(TIn) == 4 || sizeof(TOut) == 4, float, double>;
@@ -277,7 +275,7 @@ __global__ void __launch_bounds__(256) k_stage_generic(GenTopo t, HookTable H, P
     euler_direction<ND, 1, TIn, TC>(t, hk, pc, a.in, (int)c, nbr, qc, qn, dx, dt, acc);
     if constexpr (ND == 3) euler_direction<ND, 2, TIn, TC>(t, hk, pc, a.in, (int)c, nbr, qc, qn, dx, dt, acc);
   }
-  // CNS and heat: one direction at a time
+  // CNS: one direction at a time
   for (int d = 0; d < ND && PHYS != HOM3G_EULER; ++d) {
     const int m = t.nghbr[(2 * d) * t.ld + c];
     const int p = t.nghbr[(2 * d + 1) * t.ld + c];
@@ -288,32 +286,22 @@ __global__ void __launch_bounds__(256) k_stage_generic(GenTopo t, HookTable H, P
       for (int v = 0; v < NV; ++v) acc[v] = TC(__builtin_nan(""));
       continue;
     }
-    if constexpr (PHYS == HOM3G_HEAT) {
-      // heat/physics.hpp:113-119: (1/dx) * (T_l - T_r), dx of the centre cell
-      const double Tc = a.in[c];
-      const double fm = 1 / dx * (a.in[m] - Tc);
-      const double fp = 1 / dx * (Tc - a.in[p]);
-      acc[0] += (fm - fp);
-    } else {
-      TC fm[NV], fp[NV];
-      face_flux<ND, PHYS, TIn, TC>(t, hk, pc, a.in, m, (int)c, d, dx, dt, fm);
-      face_flux<ND, PHYS, TIn, TC>(t, hk, pc, a.in, (int)c, p, d, dx, dt, fp);
+    TC fm[NV], fp[NV];
+    face_flux<ND, PHYS, TIn, TC>(t, hk, pc, a.in, m, (int)c, d, dx, dt, fm);
+    face_flux<ND, PHYS, TIn, TC>(t, hk, pc, a.in, (int)c, p, d, dx, dt, fp);
 #pragma unroll
-      for (int v = 0; v < NV; ++v) acc[v] += (fm[v] - fp[v]);
-    }
+    for (int v = 0; v < NV; ++v) acc[v] += (fm[v] - fp[v]);
   }
-  const double s = (a.src != nullptr) ? dt * a.src[c] : 0.0;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const double nf = dt / dx * acc[v];
-    const double src = (v == 0 && PHYS == HOM3G_HEAT) ? s : 0.0;
     const double q = (double)a.in[v * t.ld + c];
     double o;
     switch (a.kind) {
-      case 0: o = q + nf + src; break;
+      case 0: o = q + nf; break;
       case 1: o = 0.5 * (a.base[v * t.ld + c] + q + nf); break;
-      case 2: o = 0.75 * a.base[v * t.ld + c] + 0.25 * (q + nf + src); break;
-      case 3: o = (1. / 3.) * a.base[v * t.ld + c] + (2. / 3.) * (q + nf + src); break;
+      case 2: o = 0.75 * a.base[v * t.ld + c] + 0.25 * (q + nf); break;
+      case 3: o = (1. / 3.) * a.base[v * t.ld + c] + (2. / 3.) * (q + nf); break;
       default: o = q + nf; break;
     }
     a.out[v * t.ld + c] = (TOut)o;
@@ -589,7 +577,7 @@ __global__ void __launch_bounds__(256) k_dt(const double* Q, long long ld, const
 }
 
 // set_dt (solver.hpp:541-551), on the device; resets the running minimum
-__global__ void k_set_dt(DevScalars* s, double h) {
+__device__ __forceinline__ void set_dt(DevScalars* s, double h) {
   const double dtm = ordered_to_dbl(s->dtmin);
   if (s->time + s->dt < s->tEnd) {
     s->dt = (s->step == s->forced_step) ? s->forced_dt : dtm;
@@ -603,6 +591,7 @@ __global__ void k_set_dt(DevScalars* s, double h) {
   // dt / h for the brick stages, once per step instead of once per thread
   s->dtdx = h > 0.0 ? s->dt / h : 0.0;
 }
+__global__ void k_set_dt(DevScalars* s, double h) { set_dt(s, h); }
 
 // advance (solver.hpp:502-505)
 __global__ void k_advance(DevScalars* s) {
@@ -612,18 +601,35 @@ __global__ void k_advance(DevScalars* s) {
 
 __global__ void k_reset_min(DevScalars* s) { s->dtmin = dbl_to_ordered(1.7976931348623157e308); }
 
-// coupling::apply(Tr0, cns, heat) (coupling.hpp:47-63): both minima must be
-// in dtmin of the two solvers
-__global__ void k_couple_cht(DevScalars* cns, DevScalars* heat, double scaling) {
+// coupling::apply(Tr0, cns, heat) (coupling.hpp:47-63) and both solvers'
+// set_dt: the fluid's minimum in its dtmin, the solid's bound (every cell of
+// a heat solver has the same length) as an argument; hc, hh: the cell lengths
+// of brick solvers, 0 otherwise
+__global__ void k_couple_cht(DevScalars* cns, DevScalars* heat, double scaling, double heat_min, double hc, double hh) {
   const double mc = ordered_to_dbl(cns->dtmin);
-  const double mh = ordered_to_dbl(heat->dtmin) / scaling;
-  const double dt = ref_min(mc, mh);
+  const double dt = ref_min(mc, heat_min / scaling);
   cns->forced_step = cns->step;
   cns->forced_dt = dt;
   heat->forced_step = heat->step;
   heat->forced_dt = dt * scaling;
-  cns->dtmin = dbl_to_ordered(1.7976931348623157e308);
-  heat->dtmin = dbl_to_ordered(1.7976931348623157e308);
+  set_dt(cns, hc);
+  set_dt(heat, hh);
+}
+
+// a prescribed dt for the pair's next step and both solvers' set_dt; the dts
+// they take go to rec (if any)
+__global__ void k_force_pair_dt(DevScalars* cns, DevScalars* heat, double dt, double scaling, double hc, double hh,
+                                double* rec) {
+  cns->forced_step = cns->step;
+  cns->forced_dt = dt;
+  heat->forced_step = heat->step;
+  heat->forced_dt = dt * scaling;
+  set_dt(cns, hc);
+  set_dt(heat, hh);
+  if (rec) {
+    rec[0] = cns->dt;
+    rec[1] = heat->dt;
+  }
 }
 
 // coupling::apply(s1, s2) (coupling.hpp:66-73)
@@ -851,76 +857,112 @@ void launch_stage_t(Ctx& C, SolverDev& S, const StageArgsT<TIn, TOut>& a) {
   C.prof_mark();
 }
 
-// Heat stage with FP32 stage states (FP32 flux arithmetic, FP64 RK
-// combination; the same statements as k_stage_generic's heat branch):
-// in/out are float (stage buffers) or double (lhs)
-template <int ND, class TIn, class TOut>
-__global__ void __launch_bounds__(256) k_heat_stage32(GenTopo t, const void* inv, const double* base, void* outv,
-                                                      const double* src, int kind, const DevScalars* scal) {
-  const long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (c >= t.n_int) return;
-  const TIn* in = static_cast<const TIn*>(inv);
-  const double dt = scal->dt;
-  const double dx = t.len[c];
-  const float idx = (float)(1 / dx);
-  float acc = 0.0f;
-  for (int d = 0; d < ND; ++d) {
-    const int m = t.nghbr[(2 * d) * t.ld + c];
-    const int p = t.nghbr[(2 * d + 1) * t.ld + c];
-    if (m < 0 || p < 0) {
-      acc = __builtin_nanf("");
-      continue;
-    }
-    const float Tc = (float)in[c];
-    const float fm = idx * ((float)in[m] - Tc);
-    const float fp = idx * (Tc - (float)in[p]);
-    acc += (fm - fp);
-  }
-  const double sv = (src != nullptr) ? dt * src[c] : 0.0;
-  const double nf = dt / dx * (double)acc;
-  const double q = (double)in[c];
-  double o;
-  switch (kind) {
-    case 0: o = q + nf + sv; break;
-    case 1: o = 0.5 * (base[c] + q + nf); break;
-    case 2: o = 0.75 * base[c] + 0.25 * (q + nf + sv); break;
-    case 3: o = (1. / 3.) * base[c] + (2. / 3.) * (q + nf + sv); break;
-    default: o = q + nf; break;
-  }
-  static_cast<TOut*>(outv)[c] = (TOut)o;
-}
+// Heat stage (heat/physics.hpp:113-119: the face flux (1/dx)(T_l - T_r), dx
+// of the centre cell) with the ghost fill of its input: a heat ghost has one
+// neighbour, its boundary cell, so the thread of that cell forms the ghost
+// (the formulas of k_fill_ghosts), writes it to the input's ghost slot and
+// uses it.  The solid of the coupled channel (16 k cells, 64 workgroups) is
+// launch-bound: a fill and a stage took 4.0 + 3.8 us, three of each a step.
+// TC: the flux arithmetic (FP64, or FP32 with FP32 stage states; the RK
+// combination in FP64).
+struct HeatGhosts {
+  int inline_fill;       // 0: the input's ghosts are already filled
+  const int32_t *g_apply, *g_image, *g_partner;
+  const double* g_dist;
+  const double* own_lhs;
+  int nbc;
+  struct {
+    int kind, nparams;
+    double p0, kratio, gamma;
+    const double* other;
+    long long ld;
+  } bc[kMaxBC];
+};
 
-void launch_heat_stage32(Ctx& C, SolverDev& S, const void* in, bool in32, void* out, bool out32, int kind,
-                         const double* src) {
-  auto go = [&](auto kern) {
-    C.prof_mark();
-    hipLaunchKernelGGL(kern, dim3(nblk(S.n_int)), dim3(256), 0, C.stream, make_topo(S), in,
-                       (const double*)S.lhs.p, out, src, kind, (const DevScalars*)S.scal.p);
-    H3_LAUNCH_CHECK();
-    C.prof_mark();
-  };
-  if (S.nd == 2) {
-    if (in32 && out32) go(k_heat_stage32<2, float, float>);
-    else if (in32) go(k_heat_stage32<2, float, double>);
-    else if (out32) go(k_heat_stage32<2, double, float>);
-    else go(k_heat_stage32<2, double, double>);
-  } else {
-    if (in32 && out32) go(k_heat_stage32<3, float, float>);
-    else if (in32) go(k_heat_stage32<3, float, double>);
-    else if (out32) go(k_heat_stage32<3, double, float>);
-    else go(k_heat_stage32<3, double, double>);
+template <int ND, class TC, class TIn, class TOut>
+__global__ void __launch_bounds__(256) k_heat_stage(GenTopo t, HeatGhosts G, TIn* in, const double* base, TOut* out,
+                                                    const double* src, int kind, int advance, DevScalars* scal) {
+  // the conditions in LDS: indexed per lane
+  __shared__ decltype(G.bc) bcs;
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 0; k < kMaxBC; ++k)
+      if (k < G.nbc) bcs[k] = G.bc[k];
+  }
+  __syncthreads();
+  const long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  const double dt = scal->dt;
+  if (c < t.n_int) {
+    int nbr[2 * ND];
+#pragma unroll
+    for (int k = 0; k < 2 * ND; ++k) nbr[k] = t.nghbr[k * t.ld + c];
+    const double dx = t.len[c];
+    const double Tb = (double)in[c];
+    const TC Tc = (TC)in[c];
+    const TC idx = (TC)(1 / dx);
+    auto value = [&](int o) -> TC {
+      if (o < t.n_int || !G.inline_fill) return (TC)in[o];
+      const int g = o - (int)t.n_int;
+      const int b = G.g_apply[g];
+      if (b < 0) return (TC)in[o];
+      double q = Tb;
+      switch (bcs[b].kind) {
+        case HOM3G_BC_NEUMANN: q = Tb - G.g_dist[g] * (bcs[b].nparams > 0 ? bcs[b].p0 : 0.0); break;
+        case HOM3G_BC_HEAT_NEUMANN: q = Tb - G.g_dist[g] * bcs[b].p0; break;
+        case HOM3G_BC_DIRICHLET: case HOM3G_BC_HEAT_DIRICHLET: q = 2.0 * bcs[b].p0 - Tb; break;
+        case HOM3G_BC_CHT_SOLID: {
+          const double Ts0 = G.own_lhs[c];
+          const double Tf = fluid_T(bcs[b].other, bcs[b].ld, G.g_partner[g], ND, bcs[b].gamma);
+          const double kr = bcs[b].kratio;
+          const double Ts = (kr == 1.0) ? 0.5 * (Tf + Ts0) : (Tf + kr * Ts0) / (1.0 + kr);
+          q = 2.0 * Ts - Tb;
+          break;
+        }
+        default: q = (double)in[G.g_image[g]]; break;  // periodic
+      }
+      in[o] = (TIn)q;
+      return (TC)(TIn)q;
+    };
+    TC acc = TC(0);
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      const int m = nbr[2 * d], p = nbr[2 * d + 1];
+      if (m < 0 || p < 0) {
+        // a face without a neighbour or ghost is undefined in the reference
+        // (solver.hpp:448-453); the cell is poisoned
+        acc = TC(__builtin_nan(""));
+        continue;
+      }
+      const TC fm = idx * (value(m) - Tc);
+      const TC fp = idx * (Tc - value(p));
+      acc += (fm - fp);
+    }
+    const double sv = (src != nullptr) ? dt * src[c] : 0.0;
+    const double nf = dt / dx * (double)acc;
+    double o;
+    switch (kind) {
+      case 0: o = Tb + nf + sv; break;
+      case 1: o = 0.5 * (base[c] + Tb + nf); break;
+      case 2: o = 0.75 * base[c] + 0.25 * (Tb + nf + sv); break;
+      case 3: o = (1. / 3.) * base[c] + (2. / 3.) * (Tb + nf + sv); break;
+      default: o = Tb + nf; break;
+    }
+    out[c] = (TOut)o;
+  }
+  // advance (solver.hpp:502-505) with the last stage: no stage reads time or step
+  if (advance && blockIdx.x == 0 && threadIdx.x == 0) {
+    scal->time += dt;
+    scal->step += 1;
   }
 }
 
 void launch_stage(Ctx& C, SolverDev& S, const StageArgs& a) {
   if (S.nd == 2) {
     if (S.P.physics == HOM3G_EULER) launch_stage_t<2, HOM3G_EULER>(C, S, a);
-    else if (S.P.physics == HOM3G_CNS) launch_stage_t<2, HOM3G_CNS>(C, S, a);
-    else launch_stage_t<2, HOM3G_HEAT>(C, S, a);
+    else launch_stage_t<2, HOM3G_CNS>(C, S, a);
   } else {
     if (S.P.physics == HOM3G_EULER) launch_stage_t<3, HOM3G_EULER>(C, S, a);
-    else if (S.P.physics == HOM3G_CNS) launch_stage_t<3, HOM3G_CNS>(C, S, a);
-    else launch_stage_t<3, HOM3G_HEAT>(C, S, a);
+    else launch_stage_t<3, HOM3G_CNS>(C, S, a);
   }
 }
 
@@ -936,18 +978,17 @@ void launch_stage_fp32_t(Ctx& C, SolverDev& S, const StageArgsT<TIn, TOut>& a) {
     else launch_stage_t<3, HOM3G_CNS>(C, S, a);
   }
 }
-void launch_stage_fp32(Ctx& C, SolverDev& S, const void* in, bool in32, void* out, bool out32, int kind,
-                       const double* src) {
+void launch_stage_fp32(Ctx& C, SolverDev& S, const void* in, bool in32, void* out, bool out32, int kind) {
   H3_REQUIRE(S.P.physics == HOM3G_EULER || S.P.physics == HOM3G_CNS, "Euler or CNS stage");
   const double* base = S.lhs.p;
   if (in32 && out32)
-    launch_stage_fp32_t(C, S, StageArgsT<float, float>{(const float*)in, base, (float*)out, src, kind});
+    launch_stage_fp32_t(C, S, StageArgsT<float, float>{(const float*)in, base, (float*)out, kind});
   else if (in32)
-    launch_stage_fp32_t(C, S, StageArgsT<float, double>{(const float*)in, base, (double*)out, src, kind});
+    launch_stage_fp32_t(C, S, StageArgsT<float, double>{(const float*)in, base, (double*)out, kind});
   else if (out32)
-    launch_stage_fp32_t(C, S, StageArgsT<double, float>{(const double*)in, base, (float*)out, src, kind});
+    launch_stage_fp32_t(C, S, StageArgsT<double, float>{(const double*)in, base, (float*)out, kind});
   else
-    launch_stage_fp32_t(C, S, StageArgsT<double, double>{(const double*)in, base, (double*)out, src, kind});
+    launch_stage_fp32_t(C, S, StageArgsT<double, double>{(const double*)in, base, (double*)out, kind});
 }
 
 void launch_dt(Ctx& C, SolverDev& S) {
@@ -1451,24 +1492,119 @@ static void tile_steps(Ctx& C, SolverDev& S) {
   S.dtmin_current = true;
 }
 
-// one solve() (solver.hpp:140-145); skip_dt_reduction when force_dt was just
-// applied on the device for this step; last: the caller may read the lhs
-// ghosts after this step (they hold apply_bcs of the state the step began
-// with: tiles that read no ghost leave them to the last step of a solve)
-static void solve_one(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool last = true, bool lhs_ghosts = false) {
+// the conditions whose ghosts the heat stage forms itself (the others fill
+// theirs ahead of it)
+static bool heat_inline(const SolverDev& S) {
+  for (const BCDesc& b : S.bcs)
+    switch (b.kind) {
+      case HOM3G_BC_NEUMANN: case HOM3G_BC_DIRICHLET: case HOM3G_BC_HEAT_DIRICHLET: case HOM3G_BC_HEAT_NEUMANN:
+      case HOM3G_BC_PERIODIC: break;
+      case HOM3G_BC_CHT_SOLID:
+        if (!S.partners_built) return false;
+        break;
+      default: return false;
+    }
+  return true;
+}
+
+// The stages of one heat step, the advance in the last one
+static void heat_steps(Ctx& C, SolverDev& S, bool inl) {
+  const BCTable B = make_bc_table(C, S);
+  HeatGhosts G{};
+  G.inline_fill = inl ? 1 : 0;
+  G.g_apply = S.g_applybc.p;
+  G.g_image = S.g_image.p;
+  G.g_partner = S.g_partner.p;
+  G.g_dist = S.g_dist.p;
+  G.nbc = B.nbc;
+  for (int k = 0; k < B.nbc; ++k) {
+    G.bc[k].kind = B.kind[k];
+    G.bc[k].nparams = B.nparams[k];
+    G.bc[k].p0 = B.params[k][0];
+    G.bc[k].kratio = B.kratio[k];
+    G.bc[k].gamma = B.other_gamma[k];
+    G.bc[k].other = B.other_lhs[k];
+    G.bc[k].ld = B.other_ld[k];
+  }
+  const bool f32 = S.P.precision == HOM3G_FP32_STATE;
+  const double* src = S.source.p;
+  auto go = [&](auto kern, auto* in, auto* out, int kind, const double* sr, bool last) {
+    G.own_lhs = S.lhs.p;
+    C.prof_mark();
+    hipLaunchKernelGGL(kern, dim3(nblk(S.n_int)), dim3(256), 0, C.stream, make_topo(S), G, in, (const double*)S.lhs.p,
+                       out, sr, kind, last ? 1 : 0, S.scal.p);
+    H3_LAUNCH_CHECK();
+    C.prof_mark();
+  };
+  auto fill = [&](auto* buf) {
+    if (!inl) solver_fill_ghosts(C, S, buf);
+  };
+  auto stages = [&](auto ndc) {
+    constexpr int ND = decltype(ndc)::value;
+    if (S.P.ti == HOM3G_TI_EULER_FWD) {
+      if (f32) go(k_heat_stage<ND, float, double, double>, S.lhs.p, S.rhs.p, 0, src, true);
+      else go(k_heat_stage<ND, double, double, double>, S.lhs.p, S.rhs.p, 0, src, true);
+      // lhs = rhs on the internal cells; the ghost slots keep the values of
+      // this step's apply_bcs(lhs)
+      if (S.n_ghost) {
+        hipLaunchKernelGGL(k_copy_ghosts, dim3(nblk(S.n_ghost * S.nvars)), dim3(256), 0, C.stream,
+                           (const double*)S.lhs.p, S.rhs.p, (long long)S.cap, (long long)S.n_int,
+                           (long long)S.n_ghost, S.nvars);
+        H3_LAUNCH_CHECK();
+      }
+      std::swap(S.lhs.p, S.rhs.p);
+    } else if (S.P.ti == HOM3G_TI_HEUN_RK2) {
+      if (f32) {
+        go(k_heat_stage<ND, float, double, float>, S.lhs.p, S.rhs32.p, 4, nullptr, false);
+        fill(S.rhs32.p);
+        go(k_heat_stage<ND, float, float, double>, S.rhs32.p, S.lhs.p, 1, nullptr, true);
+      } else {
+        go(k_heat_stage<ND, double, double, double>, S.lhs.p, S.rhs.p, 4, nullptr, false);
+        fill(S.rhs.p);
+        go(k_heat_stage<ND, double, double, double>, S.rhs.p, S.lhs.p, 1, nullptr, true);
+      }
+    } else if (f32) {
+      go(k_heat_stage<ND, float, double, float>, S.lhs.p, S.rhs32.p, 0, src, false);
+      fill(S.rhs32.p);
+      go(k_heat_stage<ND, float, float, float>, S.rhs32.p, S.stg32.p, 2, src, false);
+      fill(S.stg32.p);
+      go(k_heat_stage<ND, float, float, double>, S.stg32.p, S.lhs.p, 3, src, true);
+    } else {
+      go(k_heat_stage<ND, double, double, double>, S.lhs.p, S.rhs.p, 0, src, false);
+      fill(S.rhs.p);
+      go(k_heat_stage<ND, double, double, double>, S.rhs.p, S.stg.p, 2, src, false);
+      fill(S.stg.p);
+      go(k_heat_stage<ND, double, double, double>, S.stg.p, S.lhs.p, 3, src, true);
+    }
+  };
+  if (S.nd == 2) stages(std::integral_constant<int, 2>());
+  else stages(std::integral_constant<int, 3>());
+}
+
+// the cell length set_dt forms dt / h with (brick solvers)
+static double dtdx_h(const SolverDev& S) { return S.kernel == HOM3G_KERNEL_BRICK ? S.h_uniform : 0.0; }
+
+// one solve() (solver.hpp:140-145)
+static void solve_one(Ctx& C, SolverDev& S, const StepFlags& f) {
   const bool brick = (S.kernel == HOM3G_KERNEL_BRICK);
-  if (lhs_ghosts) {
-    // filled by the caller
-  } else if (S.tile_ok ? (S.tile_ghosts || last || S.P.ti == HOM3G_TI_EULER_FWD) : (!brick || S.brick_table))
+  const bool inline_heat = S.P.physics == HOM3G_HEAT && heat_inline(S);
+  if (f.lhs_ghosts || inline_heat) {
+    // filled by the caller or by the stage
+  } else if (S.tile_ok ? (S.tile_ghosts || f.last || S.P.ti == HOM3G_TI_EULER_FWD) : (!brick || S.brick_table))
     solver_fill_ghosts(C, S, S.lhs.p);
-  if (!skip_dt_reduction && !((brick || S.tile_ok) && S.dtmin_current)) {
+  if (!f.skip_dt_reduction && !((brick || S.tile_ok) && S.dtmin_current)) {
     hipLaunchKernelGGL(k_reset_min, dim3(1), dim3(1), 0, C.stream, S.scal.p);
     launch_dt(C, S);
   }
-  hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, C.stream, S.scal.p, brick ? S.h_uniform : 0.0);
-  H3_LAUNCH_CHECK();
+  if (!f.dt_set) {
+    hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, C.stream, S.scal.p, dtdx_h(S));
+    H3_LAUNCH_CHECK();
+  }
   S.dtmin_current = false;
-  const double* src = S.source.p;
+  if (S.P.physics == HOM3G_HEAT) {
+    heat_steps(C, S, inline_heat);
+    return;
+  }
   if (S.tile_ok) {
     tile_steps(C, S);
     return;
@@ -1511,12 +1647,12 @@ static void solve_one(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool last = 
       brick_stage(C, S, 3, s2, S.lhs.p, fuse, true);
     }
     S.dtmin_current = fuse;
-  } else if (S.P.precision == HOM3G_FP32_STATE && S.P.physics != HOM3G_HEAT) {
+  } else if (S.P.precision == HOM3G_FP32_STATE) {
     // table-driven Euler / CNS in FP32 state: FP32 stage buffers read and
     // written at FP32, the fluxes in FP32, the RK combination in FP64, U^n (lhs)
     // FP64; the ghosts of the stage buffers are filled in FP32
     if (S.P.ti == HOM3G_TI_EULER_FWD) {
-      launch_stage(C, S, StageArgs{S.lhs.p, S.lhs.p, S.rhs.p, src, 0});
+      launch_stage(C, S, StageArgs{S.lhs.p, S.lhs.p, S.rhs.p, 0});
       if (S.n_ghost) {
         hipLaunchKernelGGL(k_copy_ghosts, dim3(nblk(S.n_ghost * S.nvars)), dim3(256), 0, C.stream,
                            (const double*)S.lhs.p, S.rhs.p, (long long)S.cap, (long long)S.n_int,
@@ -1525,41 +1661,18 @@ static void solve_one(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool last = 
       }
       std::swap(S.lhs.p, S.rhs.p);
     } else if (S.P.ti == HOM3G_TI_HEUN_RK2) {
-      launch_stage_fp32(C, S, S.lhs.p, false, S.rhs32.p, true, 4, nullptr);
+      launch_stage_fp32(C, S, S.lhs.p, false, S.rhs32.p, true, 4);
       solver_fill_ghosts(C, S, S.rhs32.p);
-      launch_stage_fp32(C, S, S.rhs32.p, true, S.lhs.p, false, 1, nullptr);
+      launch_stage_fp32(C, S, S.rhs32.p, true, S.lhs.p, false, 1);
     } else {
-      launch_stage_fp32(C, S, S.lhs.p, false, S.rhs32.p, true, 0, src);
+      launch_stage_fp32(C, S, S.lhs.p, false, S.rhs32.p, true, 0);
       solver_fill_ghosts(C, S, S.rhs32.p);
-      launch_stage_fp32(C, S, S.rhs32.p, true, S.stg32.p, true, 2, src);
+      launch_stage_fp32(C, S, S.rhs32.p, true, S.stg32.p, true, 2);
       solver_fill_ghosts(C, S, S.stg32.p);
-      launch_stage_fp32(C, S, S.stg32.p, true, S.lhs.p, false, 3, src);
-    }
-  } else if (S.P.precision == HOM3G_FP32_STATE) {
-    // table-driven heat in FP32 state: FP32 stage buffers, FP64 lhs; the
-    // interface ghosts (CHT) are formed from both solvers' FP64 lhs
-    if (S.P.ti == HOM3G_TI_EULER_FWD) {
-      launch_heat_stage32(C, S, S.lhs.p, false, S.rhs.p, false, 0, src);
-      if (S.n_ghost) {
-        hipLaunchKernelGGL(k_copy_ghosts, dim3(nblk(S.n_ghost * S.nvars)), dim3(256), 0, C.stream,
-                           (const double*)S.lhs.p, S.rhs.p, (long long)S.cap, (long long)S.n_int,
-                           (long long)S.n_ghost, S.nvars);
-        H3_LAUNCH_CHECK();
-      }
-      std::swap(S.lhs.p, S.rhs.p);
-    } else if (S.P.ti == HOM3G_TI_HEUN_RK2) {
-      launch_heat_stage32(C, S, S.lhs.p, false, S.rhs32.p, true, 4, nullptr);
-      solver_fill_ghosts(C, S, S.rhs32.p);
-      launch_heat_stage32(C, S, S.rhs32.p, true, S.lhs.p, false, 1, nullptr);
-    } else {
-      launch_heat_stage32(C, S, S.lhs.p, false, S.rhs32.p, true, 0, src);
-      solver_fill_ghosts(C, S, S.rhs32.p);
-      launch_heat_stage32(C, S, S.rhs32.p, true, S.stg32.p, true, 2, src);
-      solver_fill_ghosts(C, S, S.stg32.p);
-      launch_heat_stage32(C, S, S.stg32.p, true, S.lhs.p, false, 3, src);
+      launch_stage_fp32(C, S, S.stg32.p, true, S.lhs.p, false, 3);
     }
   } else if (S.P.ti == HOM3G_TI_EULER_FWD) {
-    launch_stage(C, S, StageArgs{S.lhs.p, S.lhs.p, S.rhs.p, src, 0});
+    launch_stage(C, S, StageArgs{S.lhs.p, S.lhs.p, S.rhs.p, 0});
     // lhs = rhs on the internal cells; the ghost slots keep the values of
     // this step's apply_bcs(lhs)
     if (S.n_ghost) {
@@ -1570,15 +1683,15 @@ static void solve_one(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool last = 
     }
     std::swap(S.lhs.p, S.rhs.p);
   } else if (S.P.ti == HOM3G_TI_HEUN_RK2) {
-    launch_stage(C, S, StageArgs{S.lhs.p, S.lhs.p, S.rhs.p, nullptr, 4});
+    launch_stage(C, S, StageArgs{S.lhs.p, S.lhs.p, S.rhs.p, 4});
     solver_fill_ghosts(C, S, S.rhs.p);
-    launch_stage(C, S, StageArgs{S.rhs.p, S.lhs.p, S.lhs.p, nullptr, 1});
+    launch_stage(C, S, StageArgs{S.rhs.p, S.lhs.p, S.lhs.p, 1});
   } else {
-    launch_stage(C, S, StageArgs{S.lhs.p, S.lhs.p, S.rhs.p, src, 0});
+    launch_stage(C, S, StageArgs{S.lhs.p, S.lhs.p, S.rhs.p, 0});
     solver_fill_ghosts(C, S, S.rhs.p);
-    launch_stage(C, S, StageArgs{S.rhs.p, S.lhs.p, S.stg.p, src, 2});
+    launch_stage(C, S, StageArgs{S.rhs.p, S.lhs.p, S.stg.p, 2});
     solver_fill_ghosts(C, S, S.stg.p);
-    launch_stage(C, S, StageArgs{S.stg.p, S.lhs.p, S.lhs.p, src, 3});
+    launch_stage(C, S, StageArgs{S.stg.p, S.lhs.p, S.lhs.p, 3});
   }
   if (!brick) {  // the brick kernels advance in their last stage
     hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, C.stream, S.scal.p);
@@ -1586,8 +1699,13 @@ static void solve_one(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool last = 
   }
 }
 
-void solver_step(Ctx& C, SolverDev& S, bool skip_dt_reduction, bool lhs_ghosts) {
-  solve_one(C, S, skip_dt_reduction, true, lhs_ghosts);
+void solver_step(Ctx& C, SolverDev& S, const StepFlags& f) { solve_one(C, S, f); }
+
+void force_pair_dt(Ctx& C, SolverDev& cns, SolverDev& heat, double dt, double scaling, double* rec) {
+  cns.dtmin_current = heat.dtmin_current = false;
+  hipLaunchKernelGGL(k_force_pair_dt, dim3(1), dim3(1), 0, C.stream, cns.scal.p, heat.scal.p, dt, scaling, dtdx_h(cns),
+                     dtdx_h(heat), rec);
+  H3_LAUNCH_CHECK();
 }
 
 // FNV-1a over the bytes a captured step depends on
@@ -1624,12 +1742,18 @@ static bool step_graph_ok(const Ctx& C, const SolverDev& S) {
 
 void solver_solve(Ctx& C, SolverDev& S, int nsteps) {
   if (nsteps < 3 || !step_graph_ok(C, S)) {
-    for (int i = 0; i < nsteps; ++i) solve_one(C, S, false, i == nsteps - 1);
+    for (int i = 0; i < nsteps; ++i) {
+      StepFlags f;
+      f.last = i == nsteps - 1;
+      solve_one(C, S, f);
+    }
     return;
   }
   // one eager step brings the per-step flags to their steady values; the
   // same step is then captured once (capture does not run it) and replayed
-  solve_one(C, S, false, false);
+  StepFlags f;
+  f.last = false;
+  solve_one(C, S, f);
   const bool dc = S.dtmin_current;
   const uint64_t key = step_key(S);
   StepGraph& G = S.step_graph;
@@ -1638,7 +1762,7 @@ void solver_solve(Ctx& C, SolverDev& S, int nsteps) {
     hipGraph_t g = nullptr;
     H3_HIP(hipStreamBeginCapture(C.stream, hipStreamCaptureModeThreadLocal));
     try {
-      solve_one(C, S, false, false);
+      solve_one(C, S, f);
     } catch (...) {
       (void)hipStreamEndCapture(C.stream, &g);
       if (g) (void)hipGraphDestroy(g);
@@ -1666,15 +1790,19 @@ static void current_min_dt(Ctx& C, SolverDev& S) {
 }
 
 void couple_cht_step(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0) {
-  // coupling::apply: min_dt of both solvers (on their current lhs)
+  // coupling::apply: min_dt of both solvers (on their current lhs); the
+  // solid's is the same for all its cells (heat/physics.hpp:82-85)
   current_min_dt(C, cns);
-  current_min_dt(C, heat);
   cns.dtmin_current = heat.dtmin_current = false;
   const double scaling = Tr0 * cns.pc.Pr0 * cns.pc.Re0;
-  hipLaunchKernelGGL(k_couple_cht, dim3(1), dim3(1), 0, C.stream, cns.scal.p, heat.scal.p, scaling);
+  const double heat_min = heat.pc.cfl * 0.5 * (heat.h_uniform * heat.h_uniform);
+  hipLaunchKernelGGL(k_couple_cht, dim3(1), dim3(1), 0, C.stream, cns.scal.p, heat.scal.p, scaling, heat_min,
+                     dtdx_h(cns), dtdx_h(heat));
   H3_LAUNCH_CHECK();
-  solve_one(C, cns, true);
-  solve_one(C, heat, true);
+  StepFlags f;
+  f.skip_dt_reduction = f.dt_set = true;
+  solve_one(C, cns, f);
+  solve_one(C, heat, f);
 }
 
 void couple_same_step(Ctx& C, SolverDev& a, SolverDev& b) {
@@ -1683,8 +1811,10 @@ void couple_same_step(Ctx& C, SolverDev& a, SolverDev& b) {
   a.dtmin_current = b.dtmin_current = false;
   hipLaunchKernelGGL(k_couple_same, dim3(1), dim3(1), 0, C.stream, a.scal.p, b.scal.p);
   H3_LAUNCH_CHECK();
-  solve_one(C, a, true);
-  solve_one(C, b, true);
+  StepFlags f;
+  f.skip_dt_reduction = true;
+  solve_one(C, a, f);
+  solve_one(C, b, f);
 }
 
 void solver_conservation_sums(Ctx& C, SolverDev& S, double* out) {
