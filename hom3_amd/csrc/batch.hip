@@ -77,9 +77,11 @@ __global__ void k_batch_copy(const double* __restrict__ a, double* __restrict__ 
     b[i] = a[i];
 }
 
-void launch_stage(Ctx& C, BatchDev& B, int kind, const void* in, bool in32, void* out, bool out32, bool last) {
+void launch_stage(Ctx& C, BatchDev& B, int kind, const void* in, bool in32, void* out, bool out32, bool last,
+                  StepDt dt_mode = StepDt::set) {
   tile_stage(C, B.nd, tile_view(B.tiles), B.pc,
-             TileStage{in, B.U.p, out, in32, out32, (long long)B.ld, (long long)B.ld, kind, last, last}, B.scal.p,
+             TileStage{in, B.U.p, out, in32, out32, (long long)B.ld, (long long)B.ld, kind, last, last, dt_mode},
+             B.scal.p,
              (unsigned)std::min<long long>(B.grid, B.tiles.ntile));
 }
 
@@ -105,16 +107,19 @@ void drop_graph(BatchDev& B) {
 // CFL bound of the new state comes fused out of the last stage, which also
 // advances.
 void enqueue_step(Ctx& C, BatchDev& B) {
-  const int nthr = 256;
-  hipLaunchKernelGGL(k_batch_set_dt, dim3(nblk(B.ninst, nthr)), dim3(nthr), 0, C.stream, B.ninst, B.scal.p);
-  H3_LAUNCH_CHECK();
+  // SSP-RK3 stages on few tiles set the dt themselves (StepDt)
+  const bool own_dt = B.ti == HOM3G_TI_SSP_RK3 && B.tiles.ntile <= kOwnDtGroups;
+  if (!own_dt) {
+    hipLaunchKernelGGL(k_batch_set_dt, dim3(nblk(B.ninst)), dim3(256), 0, C.stream, B.ninst, B.scal.p);
+    H3_LAUNCH_CHECK();
+  }
   const bool f32 = B.precision == HOM3G_FP32_STATE;
   void* s1 = f32 ? (void*)B.S1f.p : (void*)B.S1d.p;
   void* s2 = f32 ? (void*)B.S2f.p : (void*)B.S2d.p;
   if (B.ti == HOM3G_TI_SSP_RK3) {
-    launch_stage(C, B, 0, B.U.p, false, s1, f32, false);
-    launch_stage(C, B, 2, s1, f32, s2, f32, false);
-    launch_stage(C, B, 3, s2, f32, B.U.p, false, true);
+    launch_stage(C, B, 0, B.U.p, false, s1, f32, false, own_dt ? StepDt::first : StepDt::set);
+    launch_stage(C, B, 2, s1, f32, s2, f32, false, own_dt ? StepDt::middle : StepDt::set);
+    launch_stage(C, B, 3, s2, f32, B.U.p, false, true, own_dt ? StepDt::last : StepDt::set);
   } else if (B.ti == HOM3G_TI_HEUN_RK2) {
     launch_stage(C, B, 0, B.U.p, false, s1, f32, false);
     launch_stage(C, B, 1, s1, f32, B.U.p, false, true);

@@ -45,6 +45,7 @@ struct BrickArgs {
   int kind;           // stage combination (see stepper.hip StageArgs)
   int fuse_dt;
   int advance;        // last stage of the step: also time += dt, ++step
+  StepDt dt_mode;
   const unsigned* halo;  // tiled bricks: per brick, the halo cells (see brick_table_build)
 };
 
@@ -472,6 +473,12 @@ __global__ void __launch_bounds__(BrickCfg<ND>::NT) k_brick(BrickArgs A, PhysCon
       }
     }
   }
+  // the step's dt / h (first stage: formed here by one thread)
+  if (A.dt_mode == StepDt::first && t == 0) {
+    const double dt = step_dt(scal);
+    s.red[0] = dt / A.h;
+    if (blockIdx.x == 0) step_scalars(scal, A.dt_mode, false, dt, A.h);
+  }
   __syncthreads();
 
   // 2) faces once per direction, accumulated in d-ascending order
@@ -500,7 +507,8 @@ __global__ void __launch_bounds__(BrickCfg<ND>::NT) k_brick(BrickArgs A, PhysCon
   }
 
   // 3) stage combination (FP64 accumulation of the conserved variables)
-  const double dtdx = scal->dtdx;  // dt / h, formed with dt
+  const double dtdx = A.dt_mode == StepDt::first ? s.red[0]
+                      : A.dt_mode == StepDt::set ? scal->dtdx : scal->pub_dtdx;
   double o[NV];
   const int ic = G::lin(cell);
 #pragma unroll
@@ -533,12 +541,10 @@ __global__ void __launch_bounds__(BrickCfg<ND>::NT) k_brick(BrickArgs A, PhysCon
       atomic_lower(&scal->dtmin, m);
     }
   }
-  // advance (solver.hpp:502-505) fused into the step's last stage: the stage
-  // kernels read no scalar but dt, so one thread may move time and step
-  if (A.advance && blockIdx.x == 0 && t == 0) {
-    scal->time += scal->dt;
-    scal->step += 1;
-  }
+  // the scalars, by one thread (the other workgroups of a later stage read
+  // pub_dtdx or dtdx only)
+  if (A.dt_mode != StepDt::first && blockIdx.x == 0 && t == 0)
+    step_scalars(scal, A.dt_mode, A.advance != 0, A.dt_mode == StepDt::set ? scal->dt : scal->pub_dt, A.h);
 }
 
 template <int ND, int PHYS, bool MUSCL, class TC, class TIn, class TOut>
@@ -732,7 +738,8 @@ bool brick_table_build(Ctx& C, SolverDev& S) {
 }
 
 // stage: see StageArgs kinds; in/out are the device buffers for this stage
-void brick_stage(Ctx& C, SolverDev& S, int stage, const void* in, void* out, bool fuse_dt, bool advance) {
+void brick_stage(Ctx& C, SolverDev& S, int stage, const void* in, void* out, bool fuse_dt, bool advance,
+                 StepDt dt_mode) {
   BrickArgs A;
   A.in = in;
   A.base = S.lhs.p;
@@ -745,6 +752,7 @@ void brick_stage(Ctx& C, SolverDev& S, int stage, const void* in, void* out, boo
   A.kind = stage;
   A.fuse_dt = fuse_dt ? 1 : 0;
   A.advance = advance ? 1 : 0;
+  A.dt_mode = dt_mode;
   A.halo = S.brick_table ? S.brick_halo.p : nullptr;
   const bool in32 = (in == (const void*)S.rhs32.p || in == (const void*)S.stg32.p) && in != nullptr;
   const bool out32 = (out == (void*)S.rhs32.p || out == (void*)S.stg32.p) && out != nullptr;

@@ -94,7 +94,48 @@ struct DevScalars {
   unsigned long long dtmin;  // ordered-int encoded running minimum
   double dtdx;               // dt / h on a uniform grid (brick steps), set with dt
   long long diverged_step;   // first step whose dt left [1e-300, 1e300] (utilities.hpp:73-76), -1: none
+  double pub_dt, pub_dtdx;   // the dt of the step under way, from its first stage to its last (StepDt)
 };
+
+// Where a stage kernel gets its step's dt.  SSP-RK3 on bricks and tiles needs
+// no kernel for set_dt (solver.hpp:541-551): every workgroup of the first
+// stage forms the dt from the scalars (which that launch does not change) and
+// one publishes it in pub_dt, the second stage resets the running minimum
+// (which the first read and the third lowers), and the last makes it dt and
+// advances.  A launch of its own cost 1.8 us and a gap of about 2 on small
+// grids (of 36 us a step on the 256^2 vortex), 4.7 us after large stages.
+// With many workgroups the launch is the cheaper one: the 256^3 Taylor-Green
+// step (32,768 bricks) took 0.6% longer with it, the 5 M-leaf blast (19,409
+// tiles) 3%, while 3,191 and 4,096 workgroups gained 0-1% and 6,912 tiles 5%.
+constexpr long long kOwnDtGroups = 8192;
+enum class StepDt : int { set = 0, first = 1, middle = 2, last = 3 };  // set: k_set_dt or a coupling kernel has set it
+
+__device__ __forceinline__ double step_dt(const DevScalars* s) {
+  if (s->time + s->dt < s->tEnd) return (s->step == s->forced_step) ? s->forced_dt : ordered_to_dbl(s->dtmin);
+  return s->tEnd - s->time;
+}
+// (h: the cell length of a brick solver, 0 otherwise)
+__device__ __forceinline__ void publish_dt(DevScalars* s, double dt, double h) {
+  // solution_diverged (utilities.hpp:73-76), checked by the solve driver; the
+  // end-time clamp (run_solver stops there) is not divergence
+  if (s->time + s->dt < s->tEnd && (dt < 1e-300 || dt > 1e300) && s->diverged_step < 0) s->diverged_step = s->step;
+  s->pub_dt = dt;
+  s->pub_dtdx = h > 0.0 ? dt / h : 0.0;
+}
+// one thread of the stage's launch (per instance); dt: the step's
+__device__ __forceinline__ void step_scalars(DevScalars* s, StepDt m, bool advance, double dt, double h) {
+  if (m == StepDt::first) publish_dt(s, dt, h);
+  if (m == StepDt::middle) s->dtmin = dbl_to_ordered(1.7976931348623157e308);
+  if (m == StepDt::last) {
+    s->dt = dt;
+    s->dtdx = s->pub_dtdx;
+  }
+  // advance (solver.hpp:502-505): no stage but the first reads time or step
+  if (advance) {
+    s->time += dt;
+    s->step += 1;
+  }
+}
 
 struct GridDev {
   int nd = 0;
@@ -442,7 +483,7 @@ void batch_release(BatchDev& B);
 // brick.hip
 bool brick_supported(const SolverDev& S);
 bool brick_table_build(Ctx& C, SolverDev& S);
-void brick_stage(Ctx& C, SolverDev& S, int stage, const void* in, void* out, bool fuse_dt,
-                 bool advance = false);
+void brick_stage(Ctx& C, SolverDev& S, int stage, const void* in, void* out, bool fuse_dt, bool advance,
+                 StepDt dt_mode);
 
 }  // namespace hom3g

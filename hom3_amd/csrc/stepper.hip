@@ -1451,13 +1451,14 @@ double solver_min_dt(Ctx& C, SolverDev& S) {
 
 // The stages of one step on tiles: the ghosts of a stage's input are filled
 // only where some tile reads them, the CFL bound of the new state and the
-// advance are fused into the last stage (10 launches a step before, 4 now).
-static void tile_steps(Ctx& C, SolverDev& S) {
+// advance are fused into the last stage.
+static void tile_steps(Ctx& C, SolverDev& S, bool own_dt) {
   const TileView t = tile_view(S.tile);
   const unsigned grid = tile_grid(t.ntile);
   const bool f32 = S.P.precision == HOM3G_FP32_STATE;
-  auto run = [&](const void* in, bool in32, void* out, bool out32, int kind, bool last) {
-    tile_stage(C, S.nd, t, S.pc, TileStage{in, S.lhs.p, out, in32, out32, (long long)S.cap, (long long)S.n_int, kind, last, last},
+  auto run = [&](const void* in, bool in32, void* out, bool out32, int kind, bool last, StepDt m = StepDt::set) {
+    tile_stage(C, S.nd, t, S.pc, TileStage{in, S.lhs.p, out, in32, out32, (long long)S.cap, (long long)S.n_int, kind, last, last,
+                         own_dt ? m : StepDt::set},
                S.scal.p, grid);
   };
   auto ghosts = [&](bool stg) {
@@ -1483,11 +1484,11 @@ static void tile_steps(Ctx& C, SolverDev& S) {
     ghosts(false);
     run(s1, f32, S.lhs.p, false, 1, true);
   } else {
-    run(S.lhs.p, false, s1, f32, 0, false);
+    run(S.lhs.p, false, s1, f32, 0, false, StepDt::first);
     ghosts(false);
-    run(s1, f32, s2, f32, 2, false);
+    run(s1, f32, s2, f32, 2, false, StepDt::middle);
     ghosts(true);
-    run(s2, f32, S.lhs.p, false, 3, true);
+    run(s2, f32, S.lhs.p, false, 3, true, StepDt::last);
   }
   S.dtmin_current = true;
 }
@@ -1596,7 +1597,11 @@ static void solve_one(Ctx& C, SolverDev& S, const StepFlags& f) {
     hipLaunchKernelGGL(k_reset_min, dim3(1), dim3(1), 0, C.stream, S.scal.p);
     launch_dt(C, S);
   }
-  if (!f.dt_set) {
+  // SSP-RK3 stages on few bricks or tiles set the dt themselves (StepDt)
+  const long long groups = S.tile_ok ? S.tile.ntile : S.n_int / (S.nd == 3 ? 512 : 256);
+  const bool own_dt =
+      !f.dt_set && (brick || S.tile_ok) && S.P.ti == HOM3G_TI_SSP_RK3 && groups <= kOwnDtGroups;
+  if (!f.dt_set && !own_dt) {
     hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, C.stream, S.scal.p, dtdx_h(S));
     H3_LAUNCH_CHECK();
   }
@@ -1606,7 +1611,7 @@ static void solve_one(Ctx& C, SolverDev& S, const StepFlags& f) {
     return;
   }
   if (S.tile_ok) {
-    tile_steps(C, S);
+    tile_steps(C, S, own_dt);
     return;
   }
   if (brick) {
@@ -1622,7 +1627,7 @@ static void solve_one(Ctx& C, SolverDev& S, const StepFlags& f) {
       else solver_fill_ghosts(C, S, static_cast<double*>(buf));
     };
     if (S.P.ti == HOM3G_TI_EULER_FWD) {
-      brick_stage(C, S, 0, S.lhs.p, S.rhs.p, fuse, true);
+      brick_stage(C, S, 0, S.lhs.p, S.rhs.p, fuse, true, StepDt::set);
       // lhs = rhs on the internal cells; the ghost slots keep this step's
       // apply_bcs(lhs)
       if (S.brick_table && S.n_ghost) {
@@ -1634,17 +1639,18 @@ static void solve_one(Ctx& C, SolverDev& S, const StepFlags& f) {
       std::swap(S.lhs.p, S.rhs.p);
     } else if (S.P.ti == HOM3G_TI_HEUN_RK2) {
       void* s1 = f32 ? (void*)S.rhs32.p : (void*)S.rhs.p;
-      brick_stage(C, S, 4, S.lhs.p, s1, false);
+      brick_stage(C, S, 4, S.lhs.p, s1, false, false, StepDt::set);
       ghosts(s1);
-      brick_stage(C, S, 1, s1, S.lhs.p, fuse, true);
+      brick_stage(C, S, 1, s1, S.lhs.p, fuse, true, StepDt::set);
     } else {
       void* s1 = f32 ? (void*)S.rhs32.p : (void*)S.rhs.p;
       void* s2 = f32 ? (void*)S.stg32.p : (void*)S.stg.p;
-      brick_stage(C, S, 0, S.lhs.p, s1, false);
+      auto mode = [&](StepDt m) { return own_dt ? m : StepDt::set; };
+      brick_stage(C, S, 0, S.lhs.p, s1, false, false, mode(StepDt::first));
       ghosts(s1);
-      brick_stage(C, S, 2, s1, s2, false);
+      brick_stage(C, S, 2, s1, s2, false, false, mode(StepDt::middle));
       ghosts(s2);
-      brick_stage(C, S, 3, s2, S.lhs.p, fuse, true);
+      brick_stage(C, S, 3, s2, S.lhs.p, fuse, true, mode(StepDt::last));
     }
     S.dtmin_current = fuse;
   } else if (S.P.precision == HOM3G_FP32_STATE) {

@@ -26,9 +26,9 @@
 // from the halo list to the halo states to the first face, and the two
 // barriers per direction; at 5 M leaves the stages move 4.6 TB/s (the halo
 // cells are read 1.3 times per cell on top of the compulsory bytes), 90% of
-// a device copy's rate.  FP64 holds three workgroups per CU (LDS and 164
-// VGPRs), FP32 four (106 VGPRs; held to 96 or 80 it spills and runs 13% and
-// 60% slower).
+// a device copy's rate.  FP64 holds three workgroups per CU (LDS and 168
+// VGPRs; at 174 it held two and the 0.82 M-leaf step took 0.18 ms), FP32 four
+// (115 VGPRs; held to 96 or 80 it spills and runs 13% and 60% slower).
 //
 // 2D batches (which evaluated every face from both sides too), per step:
 // 512 instances of 76.7 M cells FP64 7.05 -> 5.12 ms, FP32 states 5.59 ->
@@ -232,6 +232,7 @@ struct TileArgs {
   long long ld, ncell;
   int kind;  // 0: in+nf  1: 0.5*((base+in)+nf)  2: 0.75 base + 0.25 (in+nf)  3: 1/3 base + 2/3 (in+nf)  4: in+nf
   int fuse_dt, advance, stream;
+  StepDt dt_mode;
   DevScalars* scal;
 };
 
@@ -385,7 +386,7 @@ __device__ __forceinline__ void tile_direction(TileSmem<ND, TC>& s, const TileAr
 }
 
 template <int ND, class TC, class TIn, class TOut>
-__global__ void __launch_bounds__(T) k_tile_stage(TileArgs A, PhysConst pc) {
+__global__ void __launch_bounds__(T, ND == 3 && sizeof(TC) == 8 ? 3 : 4) k_tile_stage(TileArgs A, PhysConst pc) {
   constexpr int NV = ND + 2, NHC = TileCfg<ND>::NHC, CE = TileCfg<ND>::CE;
   __shared__ TileSmem<ND, TC> s;
   const int i = threadIdx.x;
@@ -414,7 +415,7 @@ __global__ void __launch_bounds__(T) k_tile_stage(TileArgs A, PhysConst pc) {
     const TileHdr H = A.t.hdr[tile];
     const bool has = i < H.n;
     DevScalars* S = A.scal + H.inst;
-    const double dt = S->dt;
+    double dt = A.dt_mode == StepDt::set ? S->dt : S->pub_dt;
 #pragma unroll
     for (int r = 0; r * T < NHC; ++r) {
       const int j = r * T + i;
@@ -456,6 +457,7 @@ __global__ void __launch_bounds__(T) k_tile_stage(TileArgs A, PhysConst pc) {
     }
     tile_direction<ND, ND - 1, TC, TIn>(s, A, pc, H, more0, face[ND - 1], ext[ND - 1], has, own, acc);
 
+    if (A.dt_mode == StepDt::first) dt = step_dt(S);
     const double dtdx = dt * __builtin_ldexp(H.inv_root, lev);
     double o[NV];
 #pragma unroll
@@ -488,12 +490,8 @@ __global__ void __launch_bounds__(T) k_tile_stage(TileArgs A, PhysConst pc) {
         atomic_lower(&S->dtmin, m);
       }
     }
-    // advance (solver.hpp:502-505): one tile per instance; no stage reads
-    // time or step
-    if (A.advance && H.first && i == 0) {
-      S->time += dt;
-      S->step += 1;
-    }
+    // the scalars, by one tile per instance
+    if (H.first && i == 0) step_scalars(S, A.dt_mode, A.advance != 0, dt, 0.0);
     // (no barrier here: the next tile writes the states only past this
     // tile's last closing barrier, and the reduction's values only past its
     // own barriers)
@@ -600,7 +598,7 @@ void tile_stage(Ctx& C, int nd, const TileView& t, const PhysConst& pc, const Ti
   // (FP64, 100 MB), whose arrays stay there from stage to stage
   const double bytes = (double)a.ncell * (nd + 2) * ((a.in32 ? 4 : 8) + (a.out32 ? 4 : 8) + (a.kind ? 8 : 0));
   TileArgs A{t, a.in, a.base, a.out, a.ld, a.ncell, a.kind, a.fuse_dt ? 1 : 0, a.advance ? 1 : 0,
-             bytes > 128.0 * (1 << 20) ? 1 : 0, scal};
+             bytes > 128.0 * (1 << 20) ? 1 : 0, a.dt_mode, scal};
   auto go = [&](auto kern) {
     C.prof_mark();
     hipLaunchKernelGGL(kern, dim3(grid), dim3(T), 0, C.stream, A, pc);

@@ -67,6 +67,7 @@ struct TileStage {
   int kind;
   bool fuse_dt;   // reduce the CFL bound of the new state into each instance's running minimum
   bool advance;   // last stage of the step: also time += dt, ++step of each instance
+  StepDt dt_mode;
 };
 void tile_stage(Ctx& C, int nd, const TileView& t, const PhysConst& pc, const TileStage& a, DevScalars* scal,
                 unsigned grid);
