@@ -108,7 +108,7 @@ void drop_graph(BatchDev& B) {
 // advances.
 void enqueue_step(Ctx& C, BatchDev& B) {
   // SSP-RK3 stages on few tiles set the dt themselves (StepDt)
-  const bool own_dt = B.ti == HOM3G_TI_SSP_RK3 && B.tiles.ntile <= kOwnDtGroups;
+  const bool own_dt = B.ti == HOM3G_TI_SSP_RK3 && B.tiles.ntile <= kOwnDtTiles;
   if (!own_dt) {
     hipLaunchKernelGGL(k_batch_set_dt, dim3(nblk(B.ninst)), dim3(256), 0, C.stream, B.ninst, B.scal.p);
     H3_LAUNCH_CHECK();

@@ -105,9 +105,10 @@ struct DevScalars {
 // advances.  A launch of its own cost 1.8 us and a gap of about 2 on small
 // grids (of 36 us a step on the 256^2 vortex), 4.7 us after large stages.
 // With many workgroups the launch is the cheaper one: the 256^3 Taylor-Green
-// step (32,768 bricks) took 0.6% longer with it, the 5 M-leaf blast (19,409
-// tiles) 3%, while 3,191 and 4,096 workgroups gained 0-1% and 6,912 tiles 5%.
-constexpr long long kOwnDtGroups = 8192;
+// step (32,768 bricks) took 0.6% longer without it, the 5 M-leaf blast (19,409
+// tiles) 3%, while 16,384 bricks gained 1.5%, 4,096 bricks and 3,191 tiles
+// 0-1% and 6,912 tiles 5%.
+constexpr long long kOwnDtBricks = 16384, kOwnDtTiles = 8192;
 enum class StepDt : int { set = 0, first = 1, middle = 2, last = 3 };  // set: k_set_dt or a coupling kernel has set it
 
 __device__ __forceinline__ double step_dt(const DevScalars* s) {

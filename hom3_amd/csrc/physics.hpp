@@ -92,11 +92,8 @@ __device__ __forceinline__ T esum_sq(const T* u) {
 // brick kernels (forward and reverse)
 template <int ND, class T>
 __device__ __forceinline__ void brick_prims(const T* q, T gamma, T gm1, T& p, T& ia) {
-  const T ir = dev_rcp(q[ND]);
-  T u[ND];
-#pragma unroll
-  for (int d = 0; d < ND; ++d) u[d] = q[d] * ir;
-  p = gm1 * (q[ND + 1] - T(0.5) * q[ND] * esum_sq<ND>(u));
+  // rho |u|^2 / 2 = |rho u|^2 / (2 rho)
+  p = gm1 * (q[ND + 1] - T(0.5) * esum_sq<ND>(q) * dev_rcp(q[ND]));
   ia = fast_rsq(gamma * p * q[ND]);
 }
 
@@ -351,73 +348,64 @@ __device__ __forceinline__ void ausm_flux_fast(const T* qL, T uL, T pL, T aL, T 
 // dn[v] = q_R - q_L (h times the normal gradient), dt[v][t] = the sum of the
 // two cells' central differences along tangential direction t (4h times
 // the tangential surface gradient; t over the two other directions in
-// increasing order).  Same formulas as viscous_flux with the gradient
-// scalings folded into 1/rho_s and mu / h, and the face averages
-// rho_s = S / 2, u_s = (rho u)_sum / S, T = gamma (p_L + p_R) / S
-// (S = rho_L + rho_R); results differ from the reference form by a few ULP.
+// increasing order).  The formulas of viscous_flux with
+//   S = rho_L + rho_R (rho_s = S / 2), u_s = (rho u)_sum / S,
+//   P = gamma (p_L + p_R), T = P / S,
+// arranged for few instructions (about 85 FP64 operations per face against
+// 130 with each gradient formed and scaled by itself; the 3D bricks issue
+// VALU instructions most of the time):
+//   y = (P S)^(-1/2) gives sqrt(T) = P y and 1 / S = P y^2, so two
+//   reciprocals and a square root become one inverse root and a reciprocal;
+//   h du_c/dx_D = 2 g_c / S with g_c = dn[c] - dn[rho] u_c, and
+//   h du_c/dx_k = g'_ck / (2 S) with g'_ck = dt[c][k] - dt[rho][k] u_c, so
+//   every stress is W = (mu / h) (2 / S) / Re0 times a sum of g and g' / 4;
+//   rho_s h du_k/dx_D = g_k and p_s / rho_s = (g-1)(E_sum / S - |u|^2 / 2), so
+//   h (dp - (p_s / rho_s) drho) = (g-1)(dn[E] - u . g - dn[rho] E_sum / S):
+//   the two |u|^2 terms cancel.
+// Results differ from the reference form by a few ULP.  40 steps of the 256^3
+// Taylor-Green vortex 96.6 -> 92.4 ms with their download.
 template <int ND, int D, class T>
 __device__ __forceinline__ void viscous_flux_fast(const T* qL, T pL, const T* qR, T pR, const T* dn,
                                                   const T (*dt)[ND - 1], const PhysConst& pc, T q_coef,
                                                   T inv_Re0, T inv_h, T* f) {
   const int RHO = ND, E = ND + 1;
   const T S = qL[RHO] + qR[RHO];
-  const T iS = dev_rcp(S);
-  const T rho_s = T(0.5) * S;
-  const T irs = T(2) * iS;     // 1 / rho_s
-  const T irs4 = T(0.5) * iS;  // 1 / (4 rho_s), exact
-  T u_s[ND];
-  T umag2 = T(0);
+  const T P = T(pc.gamma) * (pL + pR);
+  const T y = fast_rsq(P * S);
+  const T r = P * y;   // sqrt(T)
+  const T iS = r * y;  // 1 / S
+  const T Tm = r * r;
+  // (mu / h)(2 / S) / Re0 with Sutherland's mu = T^1.5 (1 + s) / (T + s)
+  const T c = T(2) * T(pc.sOverTrefP1) * inv_h * inv_Re0;
+  const T W = (c * r) * (Tm * iS) * dev_rcp(Tm + T(pc.sOverTref));
+  T u[ND], g[ND];
 #pragma unroll
   for (int k = 0; k < ND; ++k) {
-    u_s[k] = (qL[k] + qR[k]) * iS;
-    umag2 += u_s[k] * u_s[k];
+    u[k] = (qL[k] + qR[k]) * iS;
+    g[k] = dn[k] - dn[RHO] * u[k];
   }
-  // p_s = (g-1)(rhoE_s - rho_s |u_s|^2 / 2)
-  const T p_s = T(0.5 * pc.gm1) * ((qL[E] + qR[E]) - rho_s * umag2);
-  // h times the velocity gradients du_c/dx_sd = (G[c][sd] - G[rho][sd] u_s[c]) / rho_s:
-  // full row c = D (du_D/dx_*), column sd = D (du_*/dx_D) and the diagonal
-  T gcol[ND];  // du_k / dx_D
-#pragma unroll
-  for (int k = 0; k < ND; ++k) gcol[k] = (dn[k] - dn[RHO] * u_s[k]) * irs;
-  T grow[ND];  // du_D / dx_k
-  T diag[ND];  // du_k / dx_k
+  T X[ND], diag = T(0);
 #pragma unroll
   for (int k = 0; k < ND; ++k) {
-    if (k == D) {
-      grow[k] = gcol[D];
-      diag[k] = gcol[D];
-    } else {
-      const int t = (k < D) ? k : k - 1;
-      grow[k] = (dt[D][t] - dt[RHO][t] * u_s[D]) * irs4;
-      diag[k] = (dt[k][t] - dt[RHO][t] * u_s[k]) * irs4;
-    }
+    if (k == D) continue;
+    const int t = (k < D) ? k : k - 1;
+    X[k] = g[k] + T(0.25) * (dt[D][t] - dt[RHO][t] * u[D]);
+    diag += dt[k][t] - dt[RHO][t] * u[k];
   }
-  // h dp/dx_D = (g-1)(dn[E] - (dn[rho] |u_s|^2 + sum_k 2 rho_s u_s[k] gcol[k]) / 2)
-  T grho_umag2 = dn[RHO] * umag2;
+  // 2 du_D/dx_D - 2/3 div u
+  X[D] = T(4.0 / 3.0) * g[D] - T(1.0 / 6.0) * diag;
+  // the heat flux's (dp - (p_s / rho_s) drho) / (g-1), and u . t
+  const T es = (qL[E] + qR[E]) * iS;
+  T dp = dn[E] - dn[RHO] * es;
+  T ut = T(0);
 #pragma unroll
-  for (int k = 0; k < ND; ++k) grho_umag2 += S * u_s[k] * gcol[k];
-  const T gradP = T(pc.gm1) * (dn[E] - T(0.5) * grho_umag2);
-  // Sutherland viscosity, T = gamma * avg(p) / avg(rho)
-  const T Tm = T(pc.gamma) * (pL + pR) * iS;
-  const T mu = Tm * fast_sqrt(Tm) * T(pc.sOverTrefP1) * dev_rcp(Tm + T(pc.sOverTref));
-  const T mh = mu * inv_h;
-  // heat flux: -mu gamma/((gamma-1) Pr rho_s) (dp - p/rho drho)
-  const T q = -mh * q_coef * irs * (gradP - p_s * irs * dn[RHO]);
-  T div;
-  if constexpr (ND == 2) div = diag[0] + diag[1];
-  else div = diag[0] + (diag[1] + diag[2]);
-  div = div * T(2.0 / 3.0);
-  T fE = T(0);
-#pragma unroll
-  for (int i = 0; i < ND; ++i) {
-    T t = grow[i] + gcol[i];
-    if (i == D) t -= div;
-    t = -mh * t;
-    f[i] = inv_Re0 * t;
-    fE += u_s[i] * t;
+  for (int k = 0; k < ND; ++k) {
+    dp -= u[k] * g[k];
+    ut += u[k] * X[k];
+    f[k] = -(W * X[k]);
   }
   f[RHO] = T(0);
-  f[E] = inv_Re0 * (fE + q);
+  f[E] = -(W * (ut + (q_coef * T(pc.gm1)) * dp));
 }
 
 // Cell time step (CFL), reference formulas
