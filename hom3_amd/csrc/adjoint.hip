@@ -1758,16 +1758,16 @@ __global__ void k_force_pair(DevScalars* cs, DevScalars* hs, double dt, double s
   cs->forced_dt = dt;
   hs->forced_step = hs->step;
   hs->forced_dt = dt * scaling;
-  cs->dtmin = dbl_to_ordered(1.7976931348623157e308);
-  hs->dtmin = dbl_to_ordered(1.7976931348623157e308);
+  reset_dt(*cs);
+  reset_dt(*hs);
 }
 
 // set_dt (solver.hpp:541-551) and advance (:502-505) for the tangent run
 __global__ void k_set_dt_a(DevScalars* s) {
-  const double dtm = ordered_to_dbl(s->dtmin);
+  const double dtm = dt_minimum(*s);
   if (s->time + s->dt < s->tEnd) s->dt = (s->step == s->forced_step) ? s->forced_dt : dtm;
   else s->dt = s->tEnd - s->time;
-  s->dtmin = dbl_to_ordered(1.7976931348623157e308);
+  reset_dt(*s);
 }
 __global__ void k_advance_a(DevScalars* s) {
   s->time += s->dt;

@@ -49,7 +49,7 @@ __global__ void __launch_bounds__(kTileCells) k_batch_dt(TileView t, const doubl
     __syncthreads();
     if (threadIdx.x == 0) {
       for (int k = 1; k < kTileCells / 64; ++k) m = ref_min(m, red[k]);
-      atomic_lower(&scal[H.inst].dtmin, m);
+      lower_dt(scal[H.inst], m);
     }
     __syncthreads();
   }
@@ -60,15 +60,15 @@ __global__ void k_batch_set_dt(int n, DevScalars* s) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   DevScalars& S = s[i];
-  const double dtm = ordered_to_dbl(S.dtmin);
+  const double dtm = dt_minimum(S);
   if (S.time + S.dt < S.tEnd) S.dt = (S.step == S.forced_step) ? S.forced_dt : dtm;
   else S.dt = S.tEnd - S.time;
-  S.dtmin = dbl_to_ordered(1.7976931348623157e308);
+  reset_dt(S);
 }
 
 __global__ void k_batch_reset(int n, DevScalars* s) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) s[i].dtmin = dbl_to_ordered(1.7976931348623157e308);
+  if (i < n) reset_dt(s[i]);
 }
 
 // forward Euler's lhs = rhs copy (solver.hpp:473-476)

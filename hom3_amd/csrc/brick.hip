@@ -370,6 +370,8 @@ __global__ void __launch_bounds__(BrickCfg<ND>::NT) k_brick(BrickArgs A, PhysCon
   __shared__ Smem<ND, PHYS, MUSCL, TC> s;
 
   const int t = threadIdx.x;
+  // dt / h, read ahead of every store (a scalar load, long done when used)
+  const double dtdx_set = A.dt_mode == StepDt::set ? scal->dtdx : scal->pub_dtdx;
   const long long nb = (long long)gridDim.x;
   // XCD-aware brick order (8 XCDs, round-robin dispatch)
   long long brick = blockIdx.x;
@@ -547,8 +549,7 @@ __global__ void __launch_bounds__(BrickCfg<ND>::NT) k_brick(BrickArgs A, PhysCon
   }
 
   // 3) stage combination (FP64 accumulation of the conserved variables)
-  const double dtdx = A.dt_mode == StepDt::first ? s.red[0]
-                      : A.dt_mode == StepDt::set ? scal->dtdx : scal->pub_dtdx;
+  const double dtdx = A.dt_mode == StepDt::first ? s.red[0] : dtdx_set;
   double o[NV];
   const int ic = G::lin(cell);
 #pragma unroll
@@ -578,7 +579,7 @@ __global__ void __launch_bounds__(BrickCfg<ND>::NT) k_brick(BrickArgs A, PhysCon
     if (t == 0) {
       double m = s.red[0];
       for (int k = 1; k < NT / 64; ++k) m = ref_min(m, s.red[k]);
-      atomic_lower(&scal->dtmin, m);
+      lower_dt(*scal, m);
     }
   }
   // the scalars, by one thread (the other workgroups of a later stage read

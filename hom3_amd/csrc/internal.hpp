@@ -88,14 +88,36 @@ struct PinnedBuf {
 
 // Scalars of one solver kept in device memory so the step loop never
 // synchronises with the host (solver.hpp:406-416).
+//
+// The running CFL minimum is spread over kDtSlots places in lines of their
+// own: the workgroups that are resident first all lower it, and atomics on
+// one address serialise (about 12 ns each).  With one place they took 3.4 of
+// the 32 us of a 256^2 vortex step, 3% of a 2048^2 one and 1.5% of the
+// channel's.
+constexpr int kDtSlots = 8;
+struct alignas(128) DtSlot {
+  unsigned long long v;  // ordered-int encoded (dbl_to_ordered)
+};
 struct DevScalars {
   double dt, time, tEnd, forced_dt;
   long long step, forced_step;
-  unsigned long long dtmin;  // ordered-int encoded running minimum
   double dtdx;               // dt / h on a uniform grid (brick steps), set with dt
   long long diverged_step;   // first step whose dt left [1e-300, 1e300] (utilities.hpp:73-76), -1: none
   double pub_dt, pub_dtdx;   // the dt of the step under way, from its first stage to its last (StepDt)
+  DtSlot dtmin[kDtSlots];
 };
+__host__ __device__ __forceinline__ double dt_minimum(const DevScalars& s) {
+  unsigned long long m = s.dtmin[0].v;
+#pragma unroll
+  for (int k = 1; k < kDtSlots; ++k) m = s.dtmin[k].v < m ? s.dtmin[k].v : m;
+  return ordered_to_dbl(m);
+}
+__device__ __forceinline__ void reset_dt(DevScalars& s) {
+#pragma unroll
+  for (int k = 0; k < kDtSlots; ++k) s.dtmin[k].v = dbl_to_ordered(1.7976931348623157e308);
+}
+// by one thread of a workgroup
+__device__ __forceinline__ void lower_dt(DevScalars& s, double m) { atomic_lower(&s.dtmin[blockIdx.x % kDtSlots].v, m); }
 
 // Where a stage kernel gets its step's dt.  SSP-RK3 on bricks and tiles needs
 // no kernel for set_dt (solver.hpp:541-551): every workgroup of the first
@@ -104,15 +126,15 @@ struct DevScalars {
 // (which the first read and the third lowers), and the last makes it dt and
 // advances.  A launch of its own cost 1.8 us and a gap of about 2 on small
 // grids (of 36 us a step on the 256^2 vortex), 4.7 us after large stages.
-// With many workgroups the launch is the cheaper one: the 256^3 Taylor-Green
-// step (32,768 bricks) took 0.6% longer without it, the 5 M-leaf blast (19,409
-// tiles) 3%, while 16,384 bricks gained 1.5%, 4,096 bricks and 3,191 tiles
-// 0-1% and 6,912 tiles 5%.
-constexpr long long kOwnDtBricks = 16384, kOwnDtTiles = 8192;
+// (256^2 vortex 35.9 -> 32.3 us a step.)  With many tiles the launch is the
+// cheaper one: the 5 M-leaf blast (19,409 tiles) took 3% longer without it,
+// 6,912 tiles gained 5% and 3,191 nothing; 16,384 and 32,768 bricks, whose
+// threads do not form the dt themselves, lose nothing.
+constexpr long long kOwnDtTiles = 8192;
 enum class StepDt : int { set = 0, first = 1, middle = 2, last = 3 };  // set: k_set_dt or a coupling kernel has set it
 
 __device__ __forceinline__ double step_dt(const DevScalars* s) {
-  if (s->time + s->dt < s->tEnd) return (s->step == s->forced_step) ? s->forced_dt : ordered_to_dbl(s->dtmin);
+  if (s->time + s->dt < s->tEnd) return (s->step == s->forced_step) ? s->forced_dt : dt_minimum(*s);
   return s->tEnd - s->time;
 }
 // (h: the cell length of a brick solver, 0 otherwise)
@@ -126,7 +148,7 @@ __device__ __forceinline__ void publish_dt(DevScalars* s, double dt, double h) {
 // one thread of the stage's launch (per instance); dt: the step's
 __device__ __forceinline__ void step_scalars(DevScalars* s, StepDt m, bool advance, double dt, double h) {
   if (m == StepDt::first) publish_dt(s, dt, h);
-  if (m == StepDt::middle) s->dtmin = dbl_to_ordered(1.7976931348623157e308);
+  if (m == StepDt::middle) reset_dt(*s);
   if (m == StepDt::last) {
     s->dt = dt;
     s->dtdx = s->pub_dtdx;

@@ -495,8 +495,8 @@ __host__ __device__ __forceinline__ double ordered_to_dbl(unsigned long long o) 
   return r;
 }
 
-// Lowers the running minimum *dst (ordered encoding) to m.  Every block of a
-// launch reduces into the same address, and same-address atomics serialise
+// Lowers the running minimum *dst (ordered encoding) to m.  Many blocks of a
+// launch reduce into the same address, and same-address atomics serialise
 // in one L2 channel (about 12 ns each here: 65,536 blocks cost 0.76 ms).  The
 // minimum only falls while a launch runs (it is reset by an earlier kernel),
 // so a block whose value is not below a relaxed read of it cannot lower it

@@ -572,13 +572,13 @@ __global__ void __launch_bounds__(256) k_dt(const double* Q, long long ld, const
   if (threadIdx.x == 0) {
     double m = red[0];
     for (int k = 1; k < (int)(blockDim.x >> 6); ++k) m = ref_min(m, red[k]);
-    atomic_lower(&scal->dtmin, m);
+    lower_dt(*scal, m);
   }
 }
 
 // set_dt (solver.hpp:541-551), on the device; resets the running minimum
 __device__ __forceinline__ void set_dt(DevScalars* s, double h) {
-  const double dtm = ordered_to_dbl(s->dtmin);
+  const double dtm = dt_minimum(*s);
   if (s->time + s->dt < s->tEnd) {
     s->dt = (s->step == s->forced_step) ? s->forced_dt : dtm;
     // solution_diverged (utilities.hpp:73-76), checked by the solve driver;
@@ -587,7 +587,7 @@ __device__ __forceinline__ void set_dt(DevScalars* s, double h) {
   } else {
     s->dt = s->tEnd - s->time;
   }
-  s->dtmin = dbl_to_ordered(1.7976931348623157e308);
+  reset_dt(*s);
   // dt / h for the brick stages, once per step instead of once per thread
   s->dtdx = h > 0.0 ? s->dt / h : 0.0;
 }
@@ -599,14 +599,14 @@ __global__ void k_advance(DevScalars* s) {
   s->step += 1;
 }
 
-__global__ void k_reset_min(DevScalars* s) { s->dtmin = dbl_to_ordered(1.7976931348623157e308); }
+__global__ void k_reset_min(DevScalars* s) { reset_dt(*s); }
 
 // coupling::apply(Tr0, cns, heat) (coupling.hpp:47-63) and both solvers'
 // set_dt: the fluid's minimum in its dtmin, the solid's bound (every cell of
 // a heat solver has the same length) as an argument; hc, hh: the cell lengths
 // of brick solvers, 0 otherwise
 __global__ void k_couple_cht(DevScalars* cns, DevScalars* heat, double scaling, double heat_min, double hc, double hh) {
-  const double mc = ordered_to_dbl(cns->dtmin);
+  const double mc = dt_minimum(*cns);
   const double dt = ref_min(mc, heat_min / scaling);
   cns->forced_step = cns->step;
   cns->forced_dt = dt;
@@ -634,13 +634,13 @@ __global__ void k_force_pair_dt(DevScalars* cns, DevScalars* heat, double dt, do
 
 // coupling::apply(s1, s2) (coupling.hpp:66-73)
 __global__ void k_couple_same(DevScalars* a, DevScalars* b) {
-  const double dt = ref_min(ordered_to_dbl(a->dtmin), ordered_to_dbl(b->dtmin));
+  const double dt = ref_min(dt_minimum(*a), dt_minimum(*b));
   a->forced_step = a->step;
   a->forced_dt = dt;
   b->forced_step = b->step;
   b->forced_dt = dt;
-  a->dtmin = dbl_to_ordered(1.7976931348623157e308);
-  b->dtmin = dbl_to_ordered(1.7976931348623157e308);
+  reset_dt(*a);
+  reset_dt(*b);
 }
 
 __global__ void k_copy_ghosts(const double* from, double* to, long long ld, long long n_int, long long ng, int nv) {
@@ -1329,7 +1329,6 @@ void solver_alloc_state(Ctx& C, SolverDev& S) {
   S.host_scal = DevScalars{};
   S.host_scal.tEnd = S.P.time_end;
   S.host_scal.forced_step = -1;
-  S.host_scal.dtmin = 0;
   S.host_scal.diverged_step = -1;
   solver_push_scalars(C, S);
   hipLaunchKernelGGL(k_reset_min, dim3(1), dim3(1), 0, C.stream, S.scal.p);
@@ -1424,7 +1423,6 @@ void solver_init_time(Ctx& C, SolverDev& S) {
   S.host_scal.tEnd = S.P.time_end;
   S.host_scal.forced_dt = 0;
   S.host_scal.forced_step = -1;
-  S.host_scal.dtmin = 0;
   S.host_scal.diverged_step = -1;
   solver_push_scalars(C, S);
   hipLaunchKernelGGL(k_reset_min, dim3(1), dim3(1), 0, C.stream, S.scal.p);
@@ -1443,7 +1441,7 @@ double solver_min_dt(Ctx& C, SolverDev& S) {
   hipLaunchKernelGGL(k_reset_min, dim3(1), dim3(1), 0, C.stream, S.scal.p);
   launch_dt(C, S);
   solver_pull_scalars(C, S);
-  const double r = ordered_to_dbl(S.host_scal.dtmin);
+  const double r = dt_minimum(S.host_scal);
   hipLaunchKernelGGL(k_reset_min, dim3(1), dim3(1), 0, C.stream, S.scal.p);
   H3_LAUNCH_CHECK();
   return r;
@@ -1597,9 +1595,8 @@ static void solve_one(Ctx& C, SolverDev& S, const StepFlags& f) {
     hipLaunchKernelGGL(k_reset_min, dim3(1), dim3(1), 0, C.stream, S.scal.p);
     launch_dt(C, S);
   }
-  // SSP-RK3 stages on few bricks or tiles set the dt themselves (StepDt)
-  const bool few = S.tile_ok ? S.tile.ntile <= kOwnDtTiles : S.n_int / (S.nd == 3 ? 512 : 256) <= kOwnDtBricks;
-  const bool own_dt = !f.dt_set && (brick || S.tile_ok) && S.P.ti == HOM3G_TI_SSP_RK3 && few;
+  // SSP-RK3 stages on bricks or few tiles set the dt themselves (StepDt)
+  const bool own_dt = !f.dt_set && S.P.ti == HOM3G_TI_SSP_RK3 && (brick || (S.tile_ok && S.tile.ntile <= kOwnDtTiles));
   if (!f.dt_set && !own_dt) {
     hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, C.stream, S.scal.p, dtdx_h(S));
     H3_LAUNCH_CHECK();

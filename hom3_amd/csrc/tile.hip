@@ -487,7 +487,7 @@ __global__ void __launch_bounds__(T, ND == 3 && sizeof(TC) == 8 ? 3 : 4) k_tile_
       __syncthreads();
       if (i == 0) {
         for (int k = 1; k < T / 64; ++k) m = ref_min(m, s.red[k]);
-        atomic_lower(&S->dtmin, m);
+        lower_dt(*S, m);
       }
     }
     // the scalars, by one tile per instance
