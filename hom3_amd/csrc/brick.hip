@@ -355,7 +355,10 @@ __device__ __forceinline__ void put_prims(Smem<ND, PHYS, MUSCL, TC>& s, int i, c
   s.iar[i] = ia;
 }
 
-template <int ND, int PHYS, bool MUSCL, class TC, class TIn, class TOut, bool TABLE>
+// FIRST: the step's first stage, which forms its dt itself (StepDt::first); a
+// kernel of its own, since the code for it cost the others 4% on the 2048^2
+// vortex in FP32 states
+template <int ND, int PHYS, bool MUSCL, class TC, class TIn, class TOut, bool TABLE, bool FIRST>
 __global__ void __launch_bounds__(BrickCfg<ND>::NT) k_brick(BrickArgs A, PhysConst pc, DevScalars* scal) {
   static_assert(!(TABLE && MUSCL), "tiled bricks have halos of depth 1");
   // FP64 tiled bricks stay without: 136 VGPRs with it are one wave per SIMD
@@ -370,8 +373,12 @@ __global__ void __launch_bounds__(BrickCfg<ND>::NT) k_brick(BrickArgs A, PhysCon
   __shared__ Smem<ND, PHYS, MUSCL, TC> s;
 
   const int t = threadIdx.x;
-  // dt / h, read ahead of every store (a scalar load, long done when used)
-  const double dtdx_set = A.dt_mode == StepDt::set ? scal->dtdx : scal->pub_dtdx;
+  // first stage: one thread loads what the dt is formed from, ahead of the
+  // states (a wait for it before the barrier cost 2.5 us a step)
+  DtInputs di{};
+  if constexpr (FIRST) {
+    if (t == 0) di = load_dt_inputs(scal);
+  }
   const long long nb = (long long)gridDim.x;
   // XCD-aware brick order (8 XCDs, round-robin dispatch)
   long long brick = blockIdx.x;
@@ -505,10 +512,12 @@ __global__ void __launch_bounds__(BrickCfg<ND>::NT) k_brick(BrickArgs A, PhysCon
     }
   }
   // the step's dt / h (first stage: formed here by one thread)
-  if (A.dt_mode == StepDt::first && t == 0) {
-    const double dt = step_dt(scal);
-    s.red[0] = dt / A.h;
-    if (blockIdx.x == 0) step_scalars(scal, A.dt_mode, false, dt, A.h);
+  if constexpr (FIRST) {
+    if (t == 0) {
+      const double dt = step_dt(di);
+      s.red[0] = dt / A.h;
+      if (blockIdx.x == 0) step_scalars(scal, StepDt::first, false, dt, A.h);
+    }
   }
   __syncthreads();
 
@@ -549,7 +558,9 @@ __global__ void __launch_bounds__(BrickCfg<ND>::NT) k_brick(BrickArgs A, PhysCon
   }
 
   // 3) stage combination (FP64 accumulation of the conserved variables)
-  const double dtdx = A.dt_mode == StepDt::first ? s.red[0] : dtdx_set;
+  double dtdx;
+  if constexpr (FIRST) dtdx = s.red[0];
+  else dtdx = A.dt_mode == StepDt::set ? scal->dtdx : scal->pub_dtdx;
   double o[NV];
   const int ic = G::lin(cell);
 #pragma unroll
@@ -584,7 +595,7 @@ __global__ void __launch_bounds__(BrickCfg<ND>::NT) k_brick(BrickArgs A, PhysCon
   }
   // the scalars, by one thread (the other workgroups of a later stage read
   // pub_dtdx or dtdx only)
-  if (A.dt_mode != StepDt::first && blockIdx.x == 0 && t == 0)
+  if (!FIRST && blockIdx.x == 0 && t == 0)
     step_scalars(scal, A.dt_mode, A.advance != 0, A.dt_mode == StepDt::set ? scal->dt : scal->pub_dt, A.h);
 }
 
@@ -592,20 +603,24 @@ template <int ND, int PHYS, bool MUSCL, class TC, class TIn, class TOut>
 void launch(Ctx& C, SolverDev& S, const BrickArgs& A) {
   const long long ncell = S.n_int;
   const long long nb = ncell / BrickCfg<ND>::NT;
-  C.prof_mark();
+  auto go = [&](auto kern) {
+    C.prof_mark();
+    hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(BrickCfg<ND>::NT), 0, C.stream, A, S.pc, S.scal.p);
+    H3_LAUNCH_CHECK();
+    C.prof_mark();
+  };
+  // only a first stage reads the FP64 state
+  constexpr bool kFirst = sizeof(TIn) == 8;
+  const bool first = kFirst && A.dt_mode == StepDt::first;
   if constexpr (!MUSCL) {
     if (S.brick_table) {
-      hipLaunchKernelGGL((k_brick<ND, PHYS, MUSCL, TC, TIn, TOut, true>), dim3((unsigned)nb), dim3(BrickCfg<ND>::NT),
-                         0, C.stream, A, S.pc, S.scal.p);
-      H3_LAUNCH_CHECK();
-      C.prof_mark();
+      if (first) go(k_brick<ND, PHYS, MUSCL, TC, TIn, TOut, true, kFirst>);
+      else go(k_brick<ND, PHYS, MUSCL, TC, TIn, TOut, true, false>);
       return;
     }
   }
-  hipLaunchKernelGGL((k_brick<ND, PHYS, MUSCL, TC, TIn, TOut, false>), dim3((unsigned)nb), dim3(BrickCfg<ND>::NT), 0,
-                     C.stream, A, S.pc, S.scal.p);
-  H3_LAUNCH_CHECK();
-  C.prof_mark();
+  if (first) go(k_brick<ND, PHYS, MUSCL, TC, TIn, TOut, false, kFirst>);
+  else go(k_brick<ND, PHYS, MUSCL, TC, TIn, TOut, false, false>);
 }
 
 template <int ND, int PHYS, bool MUSCL>

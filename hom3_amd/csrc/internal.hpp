@@ -126,16 +126,42 @@ __device__ __forceinline__ void lower_dt(DevScalars& s, double m) { atomic_lower
 // (which the first read and the third lowers), and the last makes it dt and
 // advances.  A launch of its own cost 1.8 us and a gap of about 2 on small
 // grids (of 36 us a step on the 256^2 vortex), 4.7 us after large stages.
-// (256^2 vortex 35.9 -> 32.3 us a step.)  With many tiles the launch is the
-// cheaper one: the 5 M-leaf blast (19,409 tiles) took 3% longer without it,
-// 6,912 tiles gained 5% and 3,191 nothing; 16,384 and 32,768 bricks, whose
-// threads do not form the dt themselves, lose nothing.
-constexpr long long kOwnDtTiles = 8192;
+// (256^2 vortex 35.9 -> 32.3 us a step.)  With many workgroups the launch is
+// the cheaper one: 16,384 bricks (2048^2 vortex, FP32 states) took 4% longer
+// without it and 4,096 (128^3) 1%, 256 gained 10%; 19,409 tiles (5 M-leaf
+// blast) took 3% longer, 6,912 gained 5% and 3,191 nothing.
+constexpr long long kOwnDtBricks = 2048, kOwnDtTiles = 8192;
 enum class StepDt : int { set = 0, first = 1, middle = 2, last = 3 };  // set: k_set_dt or a coupling kernel has set it
 
-__device__ __forceinline__ double step_dt(const DevScalars* s) {
-  if (s->time + s->dt < s->tEnd) return (s->step == s->forced_step) ? s->forced_dt : dt_minimum(*s);
-  return s->tEnd - s->time;
+// what the step's dt is formed from: loaded ahead of its use (vector loads: a
+// wait for scalar ones would be taken with the next LDS read's)
+struct DtInputs {
+  double time, dt, tEnd, forced_dt;
+  long long step, forced_step;
+  unsigned long long m[kDtSlots];
+};
+template <class T>
+__device__ __forceinline__ T load_own(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+__device__ __forceinline__ DtInputs load_dt_inputs(const DevScalars* s) {
+  DtInputs i;
+  i.time = load_own(&s->time);
+  i.dt = load_own(&s->dt);
+  i.tEnd = load_own(&s->tEnd);
+  i.forced_dt = load_own(&s->forced_dt);
+  i.step = load_own(&s->step);
+  i.forced_step = load_own(&s->forced_step);
+#pragma unroll
+  for (int k = 0; k < kDtSlots; ++k) i.m[k] = load_own(&s->dtmin[k].v);
+  return i;
+}
+__device__ __forceinline__ double step_dt(const DtInputs& i) {
+  unsigned long long m = i.m[0];
+#pragma unroll
+  for (int k = 1; k < kDtSlots; ++k) m = i.m[k] < m ? i.m[k] : m;
+  if (i.time + i.dt < i.tEnd) return (i.step == i.forced_step) ? i.forced_dt : ordered_to_dbl(m);
+  return i.tEnd - i.time;
 }
 // (h: the cell length of a brick solver, 0 otherwise)
 __device__ __forceinline__ void publish_dt(DevScalars* s, double dt, double h) {

@@ -1595,8 +1595,9 @@ static void solve_one(Ctx& C, SolverDev& S, const StepFlags& f) {
     hipLaunchKernelGGL(k_reset_min, dim3(1), dim3(1), 0, C.stream, S.scal.p);
     launch_dt(C, S);
   }
-  // SSP-RK3 stages on bricks or few tiles set the dt themselves (StepDt)
-  const bool own_dt = !f.dt_set && S.P.ti == HOM3G_TI_SSP_RK3 && (brick || (S.tile_ok && S.tile.ntile <= kOwnDtTiles));
+  // SSP-RK3 stages on few bricks or tiles set the dt themselves (StepDt)
+  const bool few = S.tile_ok ? S.tile.ntile <= kOwnDtTiles : S.n_int / (S.nd == 3 ? 512 : 256) <= kOwnDtBricks;
+  const bool own_dt = !f.dt_set && S.P.ti == HOM3G_TI_SSP_RK3 && (brick || S.tile_ok) && few;
   if (!f.dt_set && !own_dt) {
     hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, C.stream, S.scal.p, dtdx_h(S));
     H3_LAUNCH_CHECK();

@@ -457,7 +457,7 @@ __global__ void __launch_bounds__(T, ND == 3 && sizeof(TC) == 8 ? 3 : 4) k_tile_
     }
     tile_direction<ND, ND - 1, TC, TIn>(s, A, pc, H, more0, face[ND - 1], ext[ND - 1], has, own, acc);
 
-    if (A.dt_mode == StepDt::first) dt = step_dt(S);
+    if (A.dt_mode == StepDt::first) dt = step_dt(load_dt_inputs(S));
     const double dtdx = dt * __builtin_ldexp(H.inv_root, lev);
     double o[NV];
 #pragma unroll
