@@ -19,7 +19,7 @@ TI_EULER_FWD, TI_HEUN_RK2, TI_SSP_RK3 = 0, 1, 2
 RECON_NONE, RECON_MUSCL = 0, 1
 LIM_ZERO, LIM_MINMOD, LIM_VANLEER = 0, 1, 2
 FP64, FP32_STATE = 0, 1
-KERNEL_AUTO, KERNEL_GENERIC, KERNEL_BRICK = 0, 1, 2
+KERNEL_AUTO, KERNEL_GENERIC, KERNEL_BRICK, KERNEL_TILE = 0, 1, 2, 3
 GEOM_NONE, GEOM_EDGE, GEOM_SQUARE, GEOM_SPHERE = 0, 1, 2, 3
 (BC_NEUMANN, BC_DIRICHLET, BC_ISENTROPIC_VORTEX, BC_INFLOW, BC_OUTFLOW,
  BC_ADIABATIC_NOSLIP, BC_ADIABATIC_SLIP, BC_ISOTHERMAL_NOSLIP, BC_HEAT_DIRICHLET,

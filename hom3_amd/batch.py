@@ -97,7 +97,7 @@ def four_quadrant_instances(seed, n, levels=(6, 7, 8, 9), max_extra=2):
     return out
 
 
-def build_instance(H, prm, ti="ssp_rk3", cfl=0.4, ctx=None):
+def build_instance(H, prm, ti="ssp_rk3", cfl=0.4, ctx=None, kernel="auto"):
     """One instance as an fv.Solver: MinLevel(level), refinement of the disc
     (a sphere of radius R/2 with band R/2 covers the disc), 2:1 balance,
     zero-gradient Neumann boundaries, four-quadrant initial condition."""
@@ -106,7 +106,7 @@ def build_instance(H, prm, ti="ssp_rk3", cfl=0.4, ctx=None):
         half = 0.5 * prm["radius"]
         g.refine_region(prm["level"] + prm["extra"], H.Sphere(prm["centre"], half), half)
         g.balance()
-    s = H.Solver(g, physics="euler", time_integration=ti, CFL=cfl)
+    s = H.Solver(g, physics="euler", time_integration=ti, CFL=cfl, kernel=kernel)
     H.append_bcs(s, H.euler.bc.Neumann())
     s.set_initial_condition(L.IC_FOUR_QUADRANT, prm["ic"])
     s.initialize()

@@ -367,6 +367,8 @@ int hom3g_solver_build(hom3g_ctx* ctx, int sid) {
     }
     if (S.kernel != HOM3G_KERNEL_BRICK) S.brick_table = false;
     solver_build_tiles(C, S);
+    H3_REQUIRE(S.P.kernel != HOM3G_KERNEL_TILE || S.tile_ok,
+               "tile kernel requested but the topology/physics does not allow it");
     solver_alloc_state(C, S);
   });
 }

@@ -568,7 +568,8 @@ void tile_fill(Ctx& C, const SolverDev& S, TileTab& t, long long tile0, long lon
   H3_LAUNCH_CHECK();
 }
 
-// First-order Euler AUSM on the table-driven family.  Not with the
+// First-order Euler AUSM off the bricks, unless the table-driven kernel is
+// asked for.  Not with the
 // isentropic-vortex condition (its fill rewrites boundary cells, so a CFL
 // bound fused into the last stage would be stale), host callbacks or
 // Euler-Euler coupling (their ghosts come from outside the solver), nor
@@ -576,8 +577,8 @@ void tile_fill(Ctx& C, const SolverDev& S, TileTab& t, long long tile0, long lon
 // kernel poisons such a cell).
 void solver_build_tiles(Ctx& C, SolverDev& S) {
   S.tile_ok = false;
-  if (S.kernel != HOM3G_KERNEL_GENERIC || S.P.physics != HOM3G_EULER || S.P.flux != HOM3G_FLUX_AUSM ||
-      S.P.recon != HOM3G_RECON_NONE || S.has_host_bc || S.uses_vortex_bc)
+  if (S.kernel != HOM3G_KERNEL_GENERIC || S.P.kernel == HOM3G_KERNEL_GENERIC || S.P.physics != HOM3G_EULER ||
+      S.P.flux != HOM3G_FLUX_AUSM || S.P.recon != HOM3G_RECON_NONE || S.has_host_bc || S.uses_vortex_bc)
     return;
   S.tile_ghosts = false;
   for (const BCDesc& b : S.bcs) {

@@ -496,7 +496,8 @@ class Solver:
         p.time_end = prop["timeEnd"]
         p.max_cells = int(prop["maxNoCells"])
         p.precision = {"fp64": L.FP64, "fp32": L.FP32_STATE, "fp32_state": L.FP32_STATE}[precision]
-        p.kernel = {"auto": L.KERNEL_AUTO, "generic": L.KERNEL_GENERIC, "brick": L.KERNEL_BRICK}[kernel]
+        p.kernel = {"auto": L.KERNEL_AUTO, "generic": L.KERNEL_GENERIC, "brick": L.KERNEL_BRICK,
+                    "tile": L.KERNEL_TILE}[kernel]
         self.desc = p
         self.quantities = Quantities(gamma=p.gamma, Minfty=p.Minfty, ReInfty=p.ReInfty, Pr0=p.Pr0,
                                      Sutherland0=p.Sutherland0, T0=p.T0)
@@ -631,7 +632,7 @@ class Solver:
         return n.value, f.value
 
     def kernel(self):
-        """'generic' or 'brick' (the kernel family picked at build)."""
+        """'brick', or 'generic' for the table-driven and the tile kernel (the family picked at build)."""
         k = C.c_int()
         check(lib().hom3g_solver_kernel(self.ctx.h, self.id, C.byref(k)))
         return {L.KERNEL_GENERIC: "generic", L.KERNEL_BRICK: "brick"}[k.value]

@@ -51,8 +51,11 @@ enum { HOM3G_RECON_NONE = 0, HOM3G_RECON_MUSCL = 1 };
 enum { HOM3G_LIM_ZERO = 0, HOM3G_LIM_MINMOD = 1, HOM3G_LIM_VANLEER = 2 };
 /* state precision */
 enum { HOM3G_FP64 = 0, HOM3G_FP32_STATE = 1 };
-/* kernel family: AUTO picks the brick kernel when the topology allows it */
-enum { HOM3G_KERNEL_AUTO = 0, HOM3G_KERNEL_GENERIC = 1, HOM3G_KERNEL_BRICK = 2 };
+/* kernel family: AUTO picks the brick kernel when the topology allows it,
+ * else, for first-order Euler AUSM, the tile kernel, else the table-driven
+ * one.  GENERIC forces the table-driven kernel; BRICK and TILE are errors at
+ * build where the solver does not allow them. */
+enum { HOM3G_KERNEL_AUTO = 0, HOM3G_KERNEL_GENERIC = 1, HOM3G_KERNEL_BRICK = 2, HOM3G_KERNEL_TILE = 3 };
 
 /* implicit geometries (src/geometry/implicit.hpp:39-103, Inverted :119-132) */
 enum { HOM3G_GEOM_NONE = 0, HOM3G_GEOM_EDGE = 1, HOM3G_GEOM_SQUARE = 2, HOM3G_GEOM_SPHERE = 3 };
@@ -219,7 +222,8 @@ int hom3g_solver_fine_faces(hom3g_ctx* ctx, int sid, int32_t* out, int64_t* nfin
 int hom3g_solver_counts(hom3g_ctx* ctx, int sid, int64_t* ncells, int64_t* first_ghost);
 /* nd, nvars and physics of a solver (any pointer may be NULL) */
 int hom3g_solver_info(hom3g_ctx* ctx, int sid, int* nd, int* nvars, int* physics);
-/* Kernel family chosen at build (HOM3G_KERNEL_GENERIC or _BRICK). */
+/* Kernel family chosen at build: HOM3G_KERNEL_BRICK or, on the neighbour
+ * table or tiles, _GENERIC. */
 int hom3g_solver_kernel(hom3g_ctx* ctx, int sid, int* kernel);
 /* Download the topology (column-major, ld = ncells). Any pointer may be NULL. */
 int hom3g_solver_topology(hom3g_ctx* ctx, int sid, int64_t* neighbors, int64_t* node_idx,

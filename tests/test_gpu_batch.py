@@ -61,15 +61,21 @@ def test_batch_matches_oracle(ti, graph):
 
 def test_batch_of_one_equals_solver():
     import hom3_amd as H
+    from hom3_amd.batch import build_instance
     prms, gpu, ora = make(3, 1, "ssp_rk3")
     B = H.Batch(gpu, "fp64")
     B.solve(4)
-    gpu[0].solve(4)
-    # same steps; the batch kernel's AUSM differs from the table-driven
-    # solver kernel only in rounding (primitives computed once per cell)
-    err = rel_l2(B.state(0), gpu[0].lhs[:, :gpu[0].first_gc], 2)
+    # same steps; the tiles' AUSM differs from the table-driven solver
+    # kernel only in rounding (primitives computed once per cell)
+    table = build_instance(H, prms[0], ti="ssp_rk3", cfl=0.4, kernel="generic")
+    table.solve(4)
+    err = rel_l2(B.state(0), table.lhs[:, :table.first_gc], 2)
     assert np.max(err) <= 1e-13, err
-    assert B.time(0)[2] == gpu[0].step() == 4
+    assert B.time(0)[2] == table.step() == 4
+    # the solver on tiles runs the batch's kernel on the same lists
+    tiles = build_instance(H, prms[0], ti="ssp_rk3", cfl=0.4, kernel="tile")
+    tiles.solve(4)
+    np.testing.assert_array_equal(B.state(0), tiles.lhs[:, :tiles.first_gc])
     B.close()
 
 

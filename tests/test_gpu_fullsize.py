@@ -9,8 +9,10 @@ small sizes elsewhere):
   FP32-state form stays within 1e-5 of FP64 after 20 steps;
 * 3D blast (64^3 + 2 levels, 816,824 leaves): mass and energy stay
   constant to round-off over 20 steps (coarse/fine faces telescope; the
-  outflow boundary is at rest); the persistent kernel matches the
-  table-driven one to 1e-12 and its FP32-state form stays within 1e-5;
+  outflow boundary is at rest); the solver on tiles and the batch match the
+  table-driven kernel to 1e-12, and the batch's FP32-state form stays within
+  1e-5; at 5 M leaves the solver's dt has a launch of its own and its
+  workgroups sweep several tiles;
 * CHT channel at level 7 (524,288 + 16,384 cells): adjoint dot products
   equal the FP64 tangent to 1e-9 along 2 seeded directions."""
 import numpy as np
@@ -78,25 +80,30 @@ def test_tgv256_conservation_and_fp32():
 def test_blast_fullsize_conservation_and_kernels(band, leaves):
     import hom3_amd as H
     from hom3_amd import cases
-    g, s, _ = cases.blast(H, base=6, extra=2, band=band)
-    assert s.first_gc == leaves
+    g, s, _ = cases.blast(H, base=6, extra=2, band=band, kernel="generic")
+    _, t, _ = cases.blast(H, base=6, extra=2, band=band, kernel="tile")
+    assert s.first_gc == t.first_gc == leaves
     B64 = H.Batch([s], "fp64")
     B32 = H.Batch([s], "fp32")
-    s0 = s.conservation_sums()
-    s.solve(20)
-    s1 = s.conservation_sums()
-    for v in (3, 4):
-        assert abs(s1[v] - s0[v]) <= 1e-11 * abs(s0[v]), (v, s1[v], s0[v])
+    for x in (s, t):
+        s0 = x.conservation_sums()
+        x.solve(20)
+        s1 = x.conservation_sums()
+        for v in (3, 4):
+            assert abs(s1[v] - s0[v]) <= 1e-11 * abs(s0[v]), (v, s1[v], s0[v])
     B64.solve(20)
     B32.solve(20)
     q = s.lhs[:, :s.first_gc]
+    et = rel_l2(t.lhs[:, :s.first_gc], q, 3)
     e64 = rel_l2(B64.state(0), q, 3)
     e32 = rel_l2(B32.state(0), q, 3)
-    print("blast persistent fp64 vs table-driven", e64, "fp32", e32)
+    print("blast against table-driven: solver on tiles", et, "batch fp64", e64, "fp32", e32)
+    assert 0 < np.max(et) <= 1e-12, et
     assert np.max(e64) <= 1e-12, e64
     assert np.max(e32) <= 1e-5, e32
     B64.close()
     B32.close()
+    t.close()
     s.close()
 
 

@@ -16,7 +16,7 @@ QUAD = [0.45, 0.55, 0.1, 0.2, 1.0, 1.0, -0.3, 0.1, 0.5, 0.4, 0.0, 0.0, 2.0, 1.5,
 BALL = [0.5, 0.5, 0.5, 0.3, 0.1, -0.2, 0.0, 1.0, 10.0, 0.0, 0.0, 0.1, 0.125, 0.1]
 
 
-def pair(nd, base, extra, radius, band, ti, bc, precision):
+def pair(nd, base, extra, radius, band, ti, bc, precision, kernel="tile"):
     import hom3_amd as H
     centre = [0.5, 0.4, 0.6][:nd]
     ic = (O.IC_FOUR_QUADRANT, QUAD) if nd == 2 else (O.IC_SPHERE, BALL)
@@ -42,7 +42,7 @@ def pair(nd, base, extra, radius, band, ti, bc, precision):
     o.set_ic(*ic)
     o.set_perturbation(5, 0.02)
     o.initialize()
-    s = H.Solver(g, physics="euler", time_integration=ti, CFL=0.2, kernel="generic", precision=precision)
+    s = H.Solver(g, physics="euler", time_integration=ti, CFL=0.2, kernel=kernel, precision=precision)
     H.append_bcs(s, cond[1]())
     s.set_initial_condition(*ic)
     s.set_perturbation(5, 0.02)
@@ -87,6 +87,32 @@ def test_tiles_fp32_state():
     # FP32 rounding (6e-8) of two stage states and of the fluxes per step
     assert 0 < np.max(err) <= 4 * 3 * 6e-8 * 8, err
     s.close()
+
+
+def test_generic_forces_the_table_driven_kernel():
+    """kernel="generic" runs the neighbour table's kernel on a refined grid,
+    coarse/fine faces included, and kernel="tile" (auto's choice there) the
+    tiles: the same states but for rounding, and not the same bits."""
+    import hom3_amd as H
+    _, s = pair(2, 4, 2, 0.2, 0.05, "ssp_rk3", "neumann", "fp64", kernel="auto")
+    _, t = pair(2, 4, 2, 0.2, 0.05, "ssp_rk3", "neumann", "fp64", kernel="tile")
+    for ti in TI:
+        o, g = pair(2, 4, 2, 0.2, 0.05, ti, "dirichlet" if ti == "runge_kutta_2" else "neumann", "fp64",
+                    kernel="generic")
+        o.solve(4)
+        g.solve(4)
+        n = o.first_gc
+        assert np.max(rel_l2(g.lhs[:, :n], o.get("lhs")[:, :n], 2)) <= 1e-12, ti
+    s.solve(4)
+    t.solve(4)
+    np.testing.assert_array_equal(s.lhs, t.lhs)
+    assert 0 < np.max(rel_l2(t.lhs[:, :n], g.lhs[:, :n], 2)) <= 1e-12
+    # a periodic MUSCL solver has no tiles
+    gr = H.Grid(2, [0.0] * 2, [1.0] * 2, 4)
+    m = H.Solver(gr, physics="euler", time_integration="ssp_rk3", recon="muscl", kernel="tile")
+    H.append_bcs(m, H.Periodic())
+    with pytest.raises(RuntimeError, match="tile kernel requested"):
+        m.build()
 
 
 def test_fused_dt_equals_the_reduction():
