@@ -30,9 +30,12 @@ class Batch:
         self.precision = precision
 
     def set_config(self, block, tile, grid):
+        """grid: persistent workgroups of a stage; block and tile are only
+        checked (a work item is a tile of 256 cells, taken by 256 threads)."""
         check(lib().hom3g_batch_set_config(self.ctx.h, self.id, block, tile, grid))
 
     def config(self):
+        """The launch shape that runs: threads and cells of a work item, workgroups, work items."""
         b, t, g, n = C.c_int(), C.c_int(), C.c_int(), C.c_int64()
         check(lib().hom3g_batch_get_config(self.ctx.h, self.id, C.byref(b), C.byref(t), C.byref(g), C.byref(n)))
         return dict(block=b.value, tile=t.value, grid=g.value, items=n.value)

@@ -866,13 +866,10 @@ int hom3g_batch_get_config(hom3g_ctx* ctx, int bid, int* block, int* tile, int* 
   return guarded([&] {
     Ctx& C = ctx_ref(ctx);
     BatchDev& B = batch_ref(C, bid);
-    if (block) *block = B.block;
-    if (tile) *tile = B.tile;
+    if (block) *block = kTileCells;
+    if (tile) *tile = kTileCells;
     if (grid) *grid = B.grid;
-    if (nitems) {
-      *nitems = 0;
-      for (int64_t n : B.nint) *nitems += (n + B.tile - 1) / B.tile;
-    }
+    if (nitems) *nitems = B.tiles.ntile;
   });
 }
 

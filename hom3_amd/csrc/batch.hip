@@ -223,9 +223,7 @@ void batch_create(Ctx& C, const std::vector<SolverDev*>& inst, int precision, Ba
   H3_HIP(hipGetDevice(&dev));
   H3_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   B.ncu = ncu > 0 ? ncu : 256;
-  B.block = 256;
   B.grid = B.ncu * 64;
-  B.tile = 1024;
   B.dtmin_current = false;
 }
 
@@ -234,9 +232,7 @@ void batch_set_config(Ctx& C, BatchDev& B, int block, int tile, int grid) {
   H3_REQUIRE(tile >= block, "tile must hold at least one cell per thread");
   H3_REQUIRE(grid >= 1, "grid must be positive");
   (void)C;
-  B.block = block;
   B.grid = grid;
-  B.tile = tile;
   drop_graph(B);
 }
 
@@ -279,8 +275,8 @@ void batch_autotune(Ctx& C, BatchDev& B, int* best_block, int* best_tile, int* b
     if (tmin < bms) { bms = tmin; bg = B.grid; }
   }
   batch_set_config(C, B, kTileCells, kTileCells, bg);
-  if (best_block) *best_block = B.block;
-  if (best_tile) *best_tile = B.tile;
+  if (best_block) *best_block = kTileCells;
+  if (best_tile) *best_tile = kTileCells;
   if (best_grid) *best_grid = bg;
   if (best_ms) *best_ms = bms;
 }

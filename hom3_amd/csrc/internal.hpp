@@ -358,7 +358,7 @@ struct BatchDev {
   TileTab tiles;
   DevBuf<DevScalars> scal;      // per instance
   std::vector<int64_t> off, nint;
-  int ncu = 256, block = 256, tile = 1024, grid = 1024;
+  int ncu = 256, grid = 1024;
   bool dtmin_current = false;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;

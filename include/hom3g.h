@@ -365,9 +365,10 @@ int hom3g_cht_misfit_adjoint(hom3g_ctx* ctx, int cns_sid, int heat_sid, double T
  * arithmetic, FP64 U^n and RK accumulation). */
 int hom3g_batch_create(hom3g_ctx* ctx, const int* solver_ids, int n, int precision, int* batch_id);
 /* Launch shape: grid = persistent workgroups.  block (a multiple of 64, at
- * most 512) and tile (cells per work item, at least block) are checked and
- * reported; the stages run on tiles of 256 cells with 256 threads whatever
- * they are.  Changing it drops the captured graph. */
+ * most 512) and tile (at least block) are checked and otherwise unused: a
+ * work item is a tile of 256 cells of one instance, taken by 256 threads.
+ * Changing the grid drops the captured graph.  get_config (any pointer may be
+ * NULL) reports what runs: 256, 256, the grid and the number of tiles. */
 int hom3g_batch_set_config(hom3g_ctx* ctx, int batch_id, int block, int tile, int grid);
 int hom3g_batch_get_config(hom3g_ctx* ctx, int batch_id, int* block, int* tile, int* grid, int64_t* nitems);
 /* Times stage 1 over workgroups-per-CU candidates on the current state

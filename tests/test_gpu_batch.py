@@ -95,6 +95,23 @@ def test_autotune_and_configs_do_not_change_results():
     B2.close()
 
 
+def test_config_reports_what_runs():
+    import hom3_amd as H
+    prms, gpu, ora = make(5, 5, "ssp_rk3")
+    B = H.Batch(gpu, "fp64")
+    items = sum(-(-s.first_gc // 256) for s in gpu)
+    c = B.config()
+    assert (c["block"], c["tile"], c["items"]) == (256, 256, items) and c["grid"] >= 1
+    B.set_config(64, 64, 7)
+    assert B.config() == dict(block=256, tile=256, grid=7, items=items)
+    for bad in ((63, 256, 1), (1024, 1024, 1), (256, 128, 1), (256, 256, 0)):
+        with pytest.raises(RuntimeError):
+            B.set_config(*bad)
+    a = B.autotune()
+    assert B.config() == dict(block=256, tile=256, grid=a["grid"], items=items)
+    B.close()
+
+
 def test_batch_fp32_state_error():
     """FP32 stage buffers and flux arithmetic, FP64 U^n and accumulation:
     relative L2 error against the FP64 oracle stays below 1e-5."""
