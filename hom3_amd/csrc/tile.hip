@@ -122,7 +122,9 @@ __global__ void __launch_bounds__(T) k_tile_lists(TileTopo t, TileOut o, long lo
     if (h < NHC) o.halo[tile * NHC + h] = (int32_t)(cell + o.cell0);
     else o.halo_more[H.halo0 + h - NHC] = (int32_t)(cell + o.cell0);
   };
-  if (FILL && has) o.lev[tile * T + i] = (uint8_t)ilogb(t.root / t.len[c]);  // len = root / 2^level, exact
+  // (len = root / 2^level, exact; lanes past the last cell: level 0, and below
+  // their own slots for both faces)
+  if (FILL) o.lev[tile * T + i] = has ? (uint8_t)ilogb(t.root / t.len[c]) : (uint8_t)0;
   for (int d = 0; d < ND; ++d) {
     const int lo = has ? across(t, c, 2 * d) : (int)c, up = has ? across(t, c, 2 * d + 1) : (int)c;
     if (has && (lo == kMissing || up == kMissing)) atomicOr(missing, 1);
@@ -188,6 +190,8 @@ __global__ void __launch_bounds__(T) k_tile_lists(TileTopo t, TileOut o, long lo
         if (shared) upper = (unsigned)(up - base);
         else upper = up_fine ? (kFineFlag | (unsigned)start[1]) : (unsigned)(T + start[1]);
         o.face[d * o.ldw + tile * T + i] = lower | (upper << 16);
+      } else {
+        o.face[d * o.ldw + tile * T + i] = (unsigned)i | ((unsigned)i << 16);
       }
     } else if (i == 0) {
       o.hdr[tile].ne[d] = (uint16_t)ne;
