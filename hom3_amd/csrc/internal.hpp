@@ -4,87 +4,14 @@
 #include <hip/hip_runtime.h>
 #include <memory>
 #include <mutex>
-#include <stdexcept>
 #include <string>
 #include <vector>
 
 #include "../../include/hom3g.h"
+#include "memory.hpp"
 #include "physics.hpp"
 
 namespace hom3g {
-
-struct Error : std::runtime_error {
-  int code;
-  Error(int c, const std::string& m) : std::runtime_error(m), code(c) {}
-};
-
-#define H3_HIP(expr)                                                                        \
-  do {                                                                                      \
-    hipError_t e_ = (expr);                                                                 \
-    if (e_ != hipSuccess)                                                                   \
-      throw ::hom3g::Error(HOM3G_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
-  } while (0)
-
-#define H3_REQUIRE(cond, msg) \
-  do {                        \
-    if (!(cond)) throw ::hom3g::Error(HOM3G_ERR_ARG, msg); \
-  } while (0)
-
-#define H3_LAUNCH_CHECK() H3_HIP(hipGetLastError())
-
-template <class T>
-struct DevBuf {
-  T* p = nullptr;
-  size_t n = 0;
-  DevBuf() = default;
-  DevBuf(const DevBuf&) = delete;
-  DevBuf& operator=(const DevBuf&) = delete;
-  ~DevBuf() { release(); }
-  void alloc(size_t count) {
-    if (count == n && p) return;
-    release();
-    if (count) H3_HIP(hipMalloc((void**)&p, count * sizeof(T)));
-    n = count;
-  }
-  void release() {
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    n = 0;
-  }
-  void upload(const T* h, size_t count, hipStream_t s, size_t off = 0) {
-    H3_HIP(hipMemcpyAsync(p + off, h, count * sizeof(T), hipMemcpyHostToDevice, s));
-  }
-  void download(T* h, size_t count, hipStream_t s, size_t off = 0) const {
-    H3_HIP(hipMemcpyAsync(h, p + off, count * sizeof(T), hipMemcpyDeviceToHost, s));
-  }
-};
-
-// Pinned host buffer (hipHostMalloc) for stream-ordered copies out of and
-// back into device memory; released only after the device has finished the
-// copies that may still read or write it.
-template <class T>
-struct PinnedBuf {
-  T* p = nullptr;
-  size_t n = 0;
-  PinnedBuf() = default;
-  PinnedBuf(const PinnedBuf&) = delete;
-  PinnedBuf& operator=(const PinnedBuf&) = delete;
-  ~PinnedBuf() { release(); }
-  void alloc(size_t count) {
-    if (count == n && p) return;
-    release();
-    if (count) H3_HIP(hipHostMalloc((void**)&p, count * sizeof(T), hipHostMallocDefault));
-    n = count;
-  }
-  void release() {
-    if (p) {
-      (void)hipDeviceSynchronize();
-      (void)hipHostFree(p);
-    }
-    p = nullptr;
-    n = 0;
-  }
-};
 
 // Scalars of one solver kept in device memory so the step loop never
 // synchronises with the host (solver.hpp:406-416).
@@ -362,65 +289,6 @@ struct BatchDev {
   bool dtmin_current = false;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-};
-
-// Device workspace handed out in pieces and kept between calls: the adjoint
-// takes some hundred buffers per call, and allocating and freeing each cost
-// more than the sweeps.  What exceeds kKeep is given back at the end of a
-// call, the rest with its owner.
-struct Workspace {
-  static constexpr size_t kChunk = size_t(64) << 20, kKeep = size_t(2) << 30;
-  struct Chunk {
-    DevBuf<char> buf;
-    size_t used = 0;
-  };
-  std::vector<std::unique_ptr<Chunk>> chunks;
-  void* take(size_t bytes) {
-    bytes = (bytes + 255) & ~size_t(255);
-    for (auto& c : chunks)
-      if (c->buf.n - c->used >= bytes) {
-        void* p = c->buf.p + c->used;
-        c->used += bytes;
-        return p;
-      }
-    auto c = std::make_unique<Chunk>();
-    const size_t want = bytes > kChunk ? bytes : kChunk;
-    try {
-      c->buf.alloc(want);
-    } catch (const Error&) {
-      // short of memory: what lies unused goes first
-      (void)hipGetLastError();
-      drop_unused();
-      c->buf.alloc(want);
-    }
-    c->used = bytes;
-    chunks.push_back(std::move(c));
-    return chunks.back()->buf.p;
-  }
-  void drop_unused() {
-    for (size_t k = 0; k < chunks.size();)
-      if (chunks[k]->used == 0) chunks.erase(chunks.begin() + k);
-      else ++k;
-  }
-  // bytes kept and not handed out
-  size_t spare() const {
-    size_t n = 0;
-    for (auto& c : chunks) n += c->buf.n - c->used;
-    return n;
-  }
-  // end of a call: nothing handed out is in use any more
-  void give_back() {
-    size_t total = 0;
-    for (size_t k = 0; k < chunks.size();) {
-      chunks[k]->used = 0;
-      if (total + chunks[k]->buf.n > kKeep) {
-        chunks.erase(chunks.begin() + k);
-      } else {
-        total += chunks[k]->buf.n;
-        ++k;
-      }
-    }
-  }
 };
 
 struct Ctx {
