@@ -62,6 +62,7 @@ SIGNATURES = {
     "hom3g_version": (C.c_int, []),
     "hom3g_create": (C.c_int, [_P(_vp), _i32]),
     "hom3g_destroy": (C.c_int, [_vp]),
+    "hom3g_release_memory": (C.c_int, [_vp]),
     "hom3g_synchronize": (C.c_int, [_vp]),
     "hom3g_grid_create": (C.c_int, [_vp, _i32, _P(_dbl), _P(_dbl), _i32, _i32, _P(_i32)]),
     "hom3g_grid_set_tree": (C.c_int, [_vp, _i32, _i64, _P(_i64), _P(_i64)]),

@@ -118,6 +118,7 @@ int hom3g_create(hom3g_ctx** out, int device) {
       H3_HIP(hipEventCreate(&C->ev0));
       H3_HIP(hipEventCreate(&C->ev1));
       noalloc_init(*C);
+      C->pool.enlist(device);
     } catch (...) {
       delete C;
       throw;
@@ -130,6 +131,7 @@ int hom3g_destroy(hom3g_ctx* ctx) {
   return guarded([&] {
     if (!ctx) return;
     Ctx* C = reinterpret_cast<Ctx*>(ctx);
+    C->pool.delist();
     (void)hipSetDevice(C->device);
     (void)hipStreamSynchronize(C->stream);
     for (auto& B : C->batches)
@@ -152,6 +154,14 @@ int hom3g_synchronize(hom3g_ctx* ctx) {
     Ctx& C = ctx_ref(ctx);
     set_device(C);
     H3_HIP(hipStreamSynchronize(C.stream));
+  });
+}
+
+int hom3g_release_memory(hom3g_ctx* ctx) {
+  return guarded([&] {
+    Ctx& C = ctx_ref(ctx);
+    set_device(C);
+    C.pool.release();
   });
 }
 
@@ -694,6 +704,7 @@ int hom3g_solver_destroy(hom3g_ctx* ctx, int sid) {
     set_device(C);
     solver_ref(C, sid);
     H3_HIP(hipStreamSynchronize(C.stream));
+    C.pool.forget(sid);
     C.solvers[sid].reset();
   });
 }

@@ -34,7 +34,6 @@
 #include <functional>
 #include <cstdio>
 #include <cstring>
-#include <mutex>
 
 #include "brick_geo.hpp"
 #include "dual.hpp"
@@ -2141,6 +2140,14 @@ struct RevWork {
     }
     gs.alloc(std::max<size_t>(1, 3 * (nd + 2) * (size_t)S.n_ghost));
   }
+  size_t bytes() const {
+    size_t n = hpos.n * 4 + utl.n * 4 + urng.n * sizeof(int4) + maps.wmeta.n + maps.wcoef.n * 8;
+    for (const DevBuf<double>* b : {&fl, &fr, &fg, &sb, &gs, &hs}) n += b->n * 8;
+    for (const DevBuf<int32_t>* b : {&maps.wrp, &maps.wsrc, &maps.orp, &maps.og, &maps.otl, &maps.prp, &maps.pg,
+                                     &maps.ptl})
+      n += b->n * 4;
+    return n;
+  }
   // one slot per read halo entry and variable, the entries in the order of
   // the cells they read (the brick reverse map's order); the targets are
   // the internal cells some halo entry or ghost reaches
@@ -2185,18 +2192,18 @@ struct RevWork {
   }
 };
 
-// S's reverse work, built at its first reverse sweep and kept with the
-// solver: the lists depend on its topology and conditions, which are fixed
-// when it is built, and on which solver it is coupled to
-RevWork& rev_work(Ctx& C, SolverDev& S, const SolverDev& other) {
-  if (!S.rev_work || S.rev_other != other.id) {
-    S.rev_work.reset();
-    auto w = std::make_shared<RevWork>();
+// S's reverse work, built at its first reverse sweep and kept in the pool:
+// the lists depend on its topology and conditions, which are fixed when it is
+// built, and on which solver it is coupled to (with another partner they are
+// built anew)
+std::shared_ptr<RevWork> rev_work(Ctx& C, SolverDev& S, const SolverDev& other) {
+  auto w = std::static_pointer_cast<RevWork>(C.pool.find(S.id, other.id));
+  if (!w) {
+    w = std::make_shared<RevWork>();
     w->alloc(C, S, &other);
-    S.rev_work = w;
-    S.rev_other = other.id;
+    C.pool.keep(S.id, other.id, w->bytes(), w);
   }
-  return *static_cast<RevWork*>(S.rev_work.get());
+  return w;
 }
 
 // Ibar += adjoint of the stage's face fluxes (obar: adjoint of the stage
@@ -2403,20 +2410,26 @@ const StepFlags kForcedFilled = [] { StepFlags f = kForced; f.lhs_ghosts = true;
 // the buffers from a kept workspace and the stages writing to them directly
 // they take 10.0 and 21.2 ms.
 //
-// The workspace of one adjoint call: the context's, or one of its own while
-// another thread's call holds that.  Waits for the call's work before giving
-// it back, also when an exception ends it.
+// The pool for one adjoint call.  Waits for the call's work before giving the
+// pool back, also when an exception ends it.
 struct WsUse {
   Ctx& C;
-  std::unique_lock<std::mutex> lock;
-  Workspace own;
-  explicit WsUse(Ctx& c) : C(c), lock(c.ws_lock, std::try_to_lock) {}
-  Workspace& get() { return lock.owns_lock() ? C.ws : own; }
-  ~WsUse() {
-    (void)hipStreamSynchronize(C.stream);
-    get().give_back();
-  }
+  Pool::Use use;
+  WsUse(Ctx& c, const SolverDev& a, const SolverDev& b) : C(c), use(c.pool, a.id, b.id) {}
+  ~WsUse() { (void)hipStreamSynchronize(C.stream); }
 };
+// Device memory a call may still take; below `need`, what the context keeps
+// (this pair's lists too, not yet taken) goes first
+static double free_memory(Ctx& C, double need) {
+  size_t free_b = 0, total_b = 0;
+  H3_HIP(hipMemGetInfo(&free_b, &total_b));
+  free_b += C.pool.ws.spare();
+  if ((double)free_b < need && C.pool.release(true)) {
+    H3_HIP(hipMemGetInfo(&free_b, &total_b));
+    free_b += C.pool.ws.spare();
+  }
+  return (double)free_b;
+}
 template <class T>
 struct WsBuf {
   T* p = nullptr;
@@ -2562,14 +2575,11 @@ void cht_adjoint_binomial(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, i
   const bool rk3 = cns.P.ti == HOM3G_TI_SSP_RK3;
   const long long nc = (long long)cns.nvars * cns.cap, nh = (long long)heat.nvars * heat.cap;
   const int nslot = std::min(slots, std::max(nsteps - 1, 1));
-  WsUse use(C);
-  Workspace& ws = use.get();
+  WsUse use(C, cns, heat);
+  Workspace& ws = C.pool.ws;
   {
-    size_t free_b = 0, total_b = 0;
-    H3_HIP(hipMemGetInfo(&free_b, &total_b));
-    free_b += ws.spare();
     const double need = (double)(nslot + 1 + (rk3 ? 3 : 1) + 10) * (double)(nc + nh) * sizeof(double);
-    if (need > 0.9 * (double)free_b) throw Error(HOM3G_ERR_CAPACITY, "binomial checkpoints do not fit in device memory");
+    if (need > 0.9 * free_memory(C, need / 0.9)) throw Error(HOM3G_ERR_CAPACITY, "binomial checkpoints do not fit in device memory");
   }
   // stage buffers of the step being reversed
   WsBuf<double> C0, C1, C2, H0, H1, H2;
@@ -2632,7 +2642,8 @@ void cht_adjoint_binomial(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, i
   H3_HIP(hipStreamSynchronize(C.stream));
 
   // reverse sweep
-  RevWork &Wc = rev_work(C, cns, heat), &Wh = rev_work(C, heat, cns);
+  const auto wc = rev_work(C, cns, heat), wh = rev_work(C, heat, cns);
+  RevWork &Wc = *wc, &Wh = *wh;
   WsBuf<double> Cn1, Cn, Hn1, Hn, Ic, Oc, Ih, Oh, Sbar, Cend, Hend, OS;
   for (WsBuf<double>* b : {&Cn1, &Cn, &Ic, &Oc, &Cend}) b->alloc(ws, nc);
   for (WsBuf<double>* b : {&Hn1, &Hn, &Ih, &Oh, &Sbar, &Hend}) b->alloc(ws, nh);
@@ -2747,14 +2758,12 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
   const int K = store_all ? std::max(nsteps, 1) : ckpt_every, nseg = (nsteps + K - 1) / K;
   const int KS = std::min(K, nsteps);
   const int per_step = rk3 ? 3 : 1;
-  WsUse use(C);
-  Workspace& ws = use.get();
+  WsUse use(C, cns, heat);
+  Workspace& ws = C.pool.ws;
   if (store_all) {
-    size_t free_b = 0, total_b = 0;
-    H3_HIP(hipMemGetInfo(&free_b, &total_b));
-    free_b += ws.spare();
     const double need = (double)KS * per_step * (double)(nc + nh) * sizeof(double);
-    if (need > 0.9 * (double)free_b) {
+    const double free_b = free_memory(C, need / 0.9);
+    if (need > 0.9 * free_b) {
       char msg[256];
       snprintf(msg, sizeof msg, "storing every step needs %.1f GiB of device memory, %.1f GiB free; use checkpoints",
                need / (1 << 30), free_b / double(1 << 30));
@@ -2791,11 +2800,9 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
   // short), or every stage input
   bool host_ck = false;
   if (!store_all) {
-    size_t free_b = 0, total_b = 0;
-    H3_HIP(hipMemGetInfo(&free_b, &total_b));
-    free_b += ws.spare();
     const double need = (double)nseg * (double)(nc + nh) * sizeof(double);
-    host_ck = C.ckpt_memory == HOM3G_CKPT_HOST || (C.ckpt_memory == HOM3G_CKPT_AUTO && need > 0.8 * (double)free_b);
+    host_ck = C.ckpt_memory == HOM3G_CKPT_HOST ||
+              (C.ckpt_memory == HOM3G_CKPT_AUTO && need > 0.8 * free_memory(C, need / 0.8));
   }
   std::vector<WsBuf<double>> ckC(store_all || host_ck ? 0 : nseg), ckH(store_all || host_ck ? 0 : nseg);
   std::vector<PinnedBuf<double>> hkC(host_ck ? nseg : 0), hkH(host_ck ? nseg : 0);
@@ -2853,7 +2860,8 @@ void cht_adjoint_run(Ctx& C, SolverDev& cns, SolverDev& heat, double Tr0, int ns
   H3_HIP(hipStreamSynchronize(C.stream));
 
   // reverse sweep
-  RevWork &Wc = rev_work(C, cns, heat), &Wh = rev_work(C, heat, cns);
+  const auto wc = rev_work(C, cns, heat), wh = rev_work(C, heat, cns);
+  RevWork &Wc = *wc, &Wh = *wh;
   WsBuf<double> Cn1, Cn, Hn1, Hn, Ic, Oc, Ih, Oh, Sbar, Cend, Hend, OS;
   for (WsBuf<double>* b : {&Cn1, &Cn, &Ic, &Oc}) b->alloc(ws, nc);
   for (WsBuf<double>* b : {&Hn1, &Hn, &Ih, &Oh, &Sbar}) b->alloc(ws, nh);

@@ -3,7 +3,6 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <memory>
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -263,8 +262,6 @@ struct SolverDev {
   bool tile_ok = false;         // first-order Euler stages on tiles (tile.hpp)
   bool tile_ghosts = false;     // some tile reads ghosts: filled before every stage
   TileTab tile;
-  std::shared_ptr<void> rev_work;  // index lists and work buffers of the reverse sweep (adjoint.hip)
-  int rev_other = -1;              // the coupled solver they were built with
   StepGraph step_graph;
   // host-callback boundary conditions (staging of the ghosts they fill)
   bool has_host_bc = false, host_bc_ready = false;
@@ -292,8 +289,7 @@ struct BatchDev {
 };
 
 struct Ctx {
-  Workspace ws;             // of the adjoint sweep that holds ws_lock
-  std::mutex ws_lock;
+  Pool pool;                // kept between adjoint calls
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;

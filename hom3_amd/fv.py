@@ -52,6 +52,10 @@ class Context:
     def synchronize(self):
         check(lib().hom3g_synchronize(self.h))
 
+    def release_memory(self):
+        """Frees the device memory kept from one gradient to the next."""
+        check(lib().hom3g_release_memory(self.h))
+
 
 _default_ctx = None
 

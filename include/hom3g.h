@@ -139,6 +139,11 @@ const char* hom3g_last_error(void);
 int hom3g_create(hom3g_ctx** ctx, int device);
 int hom3g_destroy(hom3g_ctx* ctx);
 int hom3g_synchronize(hom3g_ctx* ctx);
+/* Frees the device memory that the context keeps from one gradient to the
+ * next (the workspace and the reverse lists of its solvers, at most 2 GiB).
+ * Any allocation of the library on the device that runs short does so by
+ * itself; other libraries' do not. */
+int hom3g_release_memory(hom3g_ctx* ctx);
 int hom3g_version(void);
 
 /* ---- grid: grid::CartesianHSP + generation::MinLevel ----------------------

@@ -6,7 +6,7 @@
 #include <cstdlib>
 #include <map>
 #include <random>
-#include <set>
+#include <thread>
 #include <hip/hip_runtime.h>
 
 // ---- the stand-in device ------------------------------------------------------
@@ -35,6 +35,7 @@ inline hipError_t hipFree(void* p) {
   device_live.erase(i);
   return hipSuccess;
 }
+inline hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 inline hipError_t hipGetLastError() { hipError_t e = last_error; last_error = hipSuccess; return e; }
 inline const char* hipGetErrorString(hipError_t e) { return e ? "out of memory" : "success"; }
 inline hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
@@ -83,7 +84,9 @@ struct Pieces {
 
 // the buffers of one call: steps x stages states of a fluid and a solid and a
 // few small ones; returns the bytes asked for
-static size_t call(Workspace& w, size_t nc, size_t nh, int buffers) {
+static size_t call(Pool& pool, size_t nc, size_t nh, int buffers) {
+  Pool::Use use(pool, 0, 1);
+  Workspace& w = pool.ws;
   Pieces P;
   size_t sum = 0;
   auto take = [&](size_t n) {
@@ -95,7 +98,6 @@ static size_t call(Workspace& w, size_t nc, size_t nh, int buffers) {
     take(nh);
   }
   for (size_t n : {size_t(8), size_t(600), size_t(100000)}) take(n);
-  w.give_back();
   return sum;
 }
 
@@ -104,7 +106,8 @@ static size_t call(Workspace& w, size_t nc, size_t nh, int buffers) {
 // are all that it takes beyond them.
 static void at_the_limit(size_t nc, size_t nh, int buffers) {
   device_size = (size_t)((nc + nh) * (double)buffers / 0.9) + 3 * Workspace::kChunk;
-  Workspace w;
+  Pool w;
+  w.enlist(0);
   for (int pass = 0; pass < 3; ++pass) {
     device_peak = device_used;
     try {
@@ -115,6 +118,76 @@ static void at_the_limit(size_t nc, size_t nh, int buffers) {
     }
     CHECK(device_used <= Workspace::kKeep, "%zu bytes kept", device_used);
   }
+}
+
+// What a pool keeps goes when an allocation runs short, also one of another
+// context; a pool that a call of another thread holds is left alone, and a
+// call's own keeps what the call uses.
+static void short_of_memory() {
+  device_size = 4096 * MB;
+  Pool a, b, other;
+  a.enlist(0);
+  b.enlist(0);
+  other.enlist(1);
+  auto object = [](size_t n) {
+    auto p = std::make_shared<DevBuf<char>>();
+    p->alloc(n);
+    return p;
+  };
+  auto adjoint = [&](Pool& p, int cns, int heat, size_t list) {
+    Pool::Use use(p, cns, heat);
+    for (int id : {cns, heat})
+      if (!p.find(id, cns + heat - id)) p.keep(id, cns + heat - id, list, object(list));
+    for (int k = 0; k < 4; ++k) p.ws.take(100 * MB);
+  };
+  adjoint(a, 0, 1, 300 * MB);
+  adjoint(b, 0, 1, 300 * MB);
+  adjoint(other, 0, 1, 300 * MB);
+  CHECK(device_used == 3000 * MB, "%zu", device_used);
+  DevBuf<char> big;
+  big.alloc(2900 * MB);  // both pools of device 0 go, device 1's stays
+  CHECK(device_used == 3900 * MB && hipGetLastError() == hipSuccess, "%zu", device_used);
+  big.release();
+  // a call of another thread holds b
+  adjoint(a, 0, 1, 300 * MB);
+  {
+    Pool::Use use(b, 4, 5);
+    b.keep(4, 5, 300 * MB, object(300 * MB));
+    b.ws.take(100 * MB);
+    std::thread([&] {
+      DevBuf<char> x;
+      x.alloc(2600 * MB);  // a's 1000 MB go
+      CHECK(device_used == 4000 * MB, "%zu", device_used);
+      bool failed = false;
+      try {
+        DevBuf<char> y;
+        y.alloc(200 * MB);
+      } catch (const Error&) {
+        failed = true;
+      }
+      CHECK(failed && hipGetLastError() == hipSuccess, "no error, or one left for the next launch");
+    }).join();
+    CHECK(b.find(4, 5) != nullptr, "an object in use");
+    // the call's own: what it uses stays, the rest goes
+    b.keep(7, 8, 300 * MB, object(300 * MB));
+    DevBuf<char> x;
+    x.alloc(2600 * MB);
+    CHECK(b.find(4, 5) && !b.find(7, 8), "objects of the call");
+  }
+  CHECK(b.find(4, 5) != nullptr, "kept after the call");
+  b.forget(5);
+  CHECK(!b.find(4, 5), "the object of a destroyed partner");
+  CHECK(b.release() && !b.release() && device_used == 1000 * MB, "%zu", device_used);
+  CHECK(other.release() && device_used == 0, "%zu", device_used);
+  // the bound, over the workspace and the objects of all solvers
+  device_size = size_t(64) << 30;
+  for (int k = 0; k < 20; ++k) {
+    adjoint(a, 2 * k, 2 * k + 1, (k % 7 + 1) * 150 * MB);
+    CHECK(device_used <= Workspace::kKeep, "%zu bytes kept after call %d", device_used, k);
+    CHECK(a.find(2 * k, 2 * k + 1) != nullptr, "the last call's object");
+  }
+  adjoint(a, 100, 101, 3000 * MB);
+  CHECK(!a.find(100, 101) && device_used <= Workspace::kKeep, "an object above the bound");
 }
 
 int main() {
@@ -130,7 +203,8 @@ int main() {
   std::mt19937 rng(5);
   for (int round = 0; round < 200; ++round) {
     device_size = size_t(64) << 30;
-    Workspace w;
+    Pool w;
+    w.enlist(0);
     for (int k = 0; k < 6; ++k) {
       const size_t nc = size_t(1) << std::uniform_int_distribution<int>(10, 29)(rng);
       call(w, nc + rng() % 5000, nc / (1 + rng() % 64) + 8, 1 + rng() % 12);
@@ -144,6 +218,8 @@ int main() {
       CHECK(false, "after other calls: %s", e.what());
     }
   }
+  CHECK(device_used == 0, "%zu bytes lost", device_used);
+  short_of_memory();
   CHECK(device_used == 0, "%zu bytes lost", device_used);
   std::printf("%d failures\n", failures);
   return failures ? 1 : 0;

@@ -31,3 +31,31 @@ def test_interleaved_calls_share_the_workspace():
         J0, g0 = ref[(level, seed, 0)]
         assert J == J0
         np.testing.assert_array_equal(g, g0)
+
+
+def test_memory_kept_between_gradients_is_given_back():
+    """release_memory frees what the gradient left on the device, and the next
+    gradient has the same bits."""
+    import torch
+    import hom3_amd as H
+
+    def used():
+        ctx.synchronize()
+        free, total = torch.cuda.mem_get_info(0)
+        return total - free
+
+    ctx = H.Context(0)
+    pair, J0, g0 = gradient(ctx, 5, 3, 0)
+    kept = used()
+    ctx.release_memory()
+    released = used()
+    # the workspace alone is one chunk of 64 MiB at least
+    assert kept - released >= 64 << 20, (kept, released)
+    _, J1, g1 = gradient(ctx, 5, 3, 0, pair)
+    assert J0 == J1
+    np.testing.assert_array_equal(g0, g1)
+    assert used() - released >= 64 << 20
+    ctx.release_memory()
+    ctx.release_memory()
+    # (the runtime's own allocations may grow by less than a chunk)
+    assert used() - released < 16 << 20

@@ -1,5 +1,6 @@
 """Bookkeeping of device memory (hom3_amd/csrc/memory.hpp): what the adjoint's
-workspace takes at the limit of a device, over calls of many sizes.
+workspace takes at the limit of a device, over calls of many sizes, and what
+becomes of the memory kept between calls when another allocation runs short.
 Host-only: tests/cpp/memory_check.cpp is compiled with g++ against a stand-in
 for the HIP allocation calls."""
 import os
