@@ -365,21 +365,26 @@ int hom3g_solver_build(hom3g_ctx* ctx, int sid) {
     SolverDev& S = solver_ref(C, sid);
     H3_REQUIRE(!S.built, "solver already built");
     GridDev& G = grid_ref(C, S.grid_id);
-    solver_build(C, G, S);
-    // kernel family
-    if (S.P.kernel == HOM3G_KERNEL_BRICK) {
-      H3_REQUIRE(S.brick_ok, "brick kernel requested but the topology/physics does not allow it");
-      S.kernel = HOM3G_KERNEL_BRICK;
-    } else if (S.P.kernel == HOM3G_KERNEL_AUTO && S.brick_ok) {
-      S.kernel = HOM3G_KERNEL_BRICK;
-    } else {
-      S.kernel = HOM3G_KERNEL_GENERIC;
+    try {
+      solver_build(C, G, S);
+      // kernel family
+      if (S.P.kernel == HOM3G_KERNEL_BRICK) {
+        H3_REQUIRE(S.brick_ok, "brick kernel requested but the topology/physics does not allow it");
+        S.kernel = HOM3G_KERNEL_BRICK;
+      } else if (S.P.kernel == HOM3G_KERNEL_AUTO && S.brick_ok) {
+        S.kernel = HOM3G_KERNEL_BRICK;
+      } else {
+        S.kernel = HOM3G_KERNEL_GENERIC;
+      }
+      if (S.kernel != HOM3G_KERNEL_BRICK) S.brick_table = false;
+      solver_alloc_state(C, S);
+      solver_build_tiles(C, S);
+      H3_REQUIRE(S.P.kernel != HOM3G_KERNEL_TILE || S.tile_ok,
+                 "tile kernel requested but the topology/physics does not allow it");
+    } catch (...) {
+      S.built = false;  // no call runs on a solver without its tables or states
+      throw;
     }
-    if (S.kernel != HOM3G_KERNEL_BRICK) S.brick_table = false;
-    solver_build_tiles(C, S);
-    H3_REQUIRE(S.P.kernel != HOM3G_KERNEL_TILE || S.tile_ok,
-               "tile kernel requested but the topology/physics does not allow it");
-    solver_alloc_state(C, S);
   });
 }
 

@@ -190,7 +190,7 @@ void batch_create(Ctx& C, const std::vector<SolverDev*>& inst, int precision, Ba
   }
   tile0[B.ninst] = (long long)hdr.size();
   H3_REQUIRE(tile0[B.ninst] * kTileCells < INT32_MAX / 2, "too many cells in the batch for 32-bit ids");
-  tile_place(C, B.nd, hdr, B.tiles);
+  H3_REQUIRE(tile_place(C, B.nd, hdr, B.tiles), "too many tile faces in the batch for 32-bit offsets");
   B.ncell = N;
   B.ld = B.tiles.ntile * kTileCells;
   const int nv = B.nvars;

@@ -208,6 +208,13 @@ struct TileTab {
   DevBuf<uint8_t> lev;
   DevBuf<int32_t> halo, halo_more;
   long long ntile = 0;
+  void release() {
+    hdr.release();
+    for (DevBuf<uint32_t>* b : {&face, &ext, &ext_more}) b->release();
+    lev.release();
+    for (DevBuf<int32_t>* b : {&halo, &halo_more}) b->release();
+    ntile = 0;
+  }
 };
 
 struct SolverDev {

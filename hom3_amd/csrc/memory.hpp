@@ -18,6 +18,11 @@ struct Error : std::runtime_error {
   Error(int c, const std::string& m) : std::runtime_error(m), code(c) {}
 };
 
+// device memory ran out (after what is kept between calls was freed)
+struct OutOfMemory : Error {
+  explicit OutOfMemory(size_t bytes) : Error(HOM3G_ERR_HIP, "out of device memory: " + std::to_string(bytes) + " bytes") {}
+};
+
 #define H3_HIP(expr)                                                                        \
   do {                                                                                      \
     hipError_t e_ = (expr);                                                                 \
@@ -37,16 +42,18 @@ struct Error : std::runtime_error {
 inline bool release_idle(int device);
 
 // hipMalloc; short of memory, what is kept goes first
-inline hipError_t device_malloc(void** p, size_t bytes) {
+inline void device_malloc(void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
     int device = 0;
     if (hipGetDevice(&device) == hipSuccess && release_idle(device)) e = hipMalloc(p, bytes);
-    // (a failed allocation is reported here and not by the next launch)
-    if (e == hipErrorOutOfMemory) (void)hipGetLastError();
   }
-  return e;
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();  // reported here and not by the next launch
+    throw OutOfMemory(bytes);
+  }
+  H3_HIP(e);
 }
 
 template <class T>
@@ -60,7 +67,7 @@ struct DevBuf {
   void alloc(size_t count) {
     if (count == n && p) return;
     release();
-    if (count) H3_HIP(device_malloc((void**)&p, count * sizeof(T)));
+    if (count) device_malloc((void**)&p, count * sizeof(T));
     n = count;
   }
   void release() {

@@ -543,7 +543,7 @@ bool tile_count(Ctx& C, const SolverDev& S, std::vector<TileHdr>& hdr, int inst)
   return true;
 }
 
-void tile_place(Ctx& C, int nd, std::vector<TileHdr>& hdr, TileTab& t) {
+bool tile_place(Ctx& C, int nd, std::vector<TileHdr>& hdr, TileTab& t) {
   const int NHC = nd == 2 ? TileCfg<2>::NHC : TileCfg<3>::NHC, CE = nd == 2 ? TileCfg<2>::CE : TileCfg<3>::CE;
   long long nh = 0, ne = 0;
   for (TileHdr& H : hdr) {
@@ -552,7 +552,7 @@ void tile_place(Ctx& C, int nd, std::vector<TileHdr>& hdr, TileTab& t) {
     nh += std::max(0, (int)H.nh - NHC);
     for (int d = 0; d < nd; ++d) ne += std::max(0, (int)H.ne[d] - CE);
   }
-  H3_REQUIRE(nh < INT32_MAX && ne < INT32_MAX, "too many tile faces for 32-bit offsets");
+  if (nh >= INT32_MAX || ne >= INT32_MAX) return false;
   t.ntile = (long long)hdr.size();
   t.hdr.alloc(hdr.size());
   t.hdr.upload(hdr.data(), hdr.size(), C.stream);
@@ -563,6 +563,7 @@ void tile_place(Ctx& C, int nd, std::vector<TileHdr>& hdr, TileTab& t) {
   t.halo_more.alloc(std::max<long long>(1, nh));
   t.ext_more.alloc(std::max<long long>(1, ne));
   H3_HIP(hipStreamSynchronize(C.stream));
+  return true;
 }
 
 void tile_fill(Ctx& C, const SolverDev& S, TileTab& t, long long tile0, long long n) {
@@ -595,8 +596,14 @@ void solver_build_tiles(Ctx& C, SolverDev& S) {
     if (b.kind != HOM3G_BC_PERIODIC && !zero_gradient(b)) S.tile_ghosts = true;
   }
   std::vector<TileHdr> hdr;
-  if (!tile_count(C, S, hdr, 0)) return;
-  tile_place(C, S.nd, hdr, S.tile);
+  try {
+    if (!tile_count(C, S, hdr, 0) || !tile_place(C, S.nd, hdr, S.tile)) return;
+  } catch (const OutOfMemory&) {
+    // the lists are 27 B per cell on top of the solver's tables and states,
+    // which are in place: it steps without them
+    S.tile.release();
+    return;
+  }
   tile_fill(C, S, S.tile, 0, S.tile.ntile);
   S.tile_ok = true;
 }

@@ -50,8 +50,9 @@ inline unsigned tile_grid(long long ntile) { return (unsigned)(ntile < 64 * 256 
 // Appends the headers of S's tiles (lists not yet placed) with their list lengths; false if some cell has a side without
 // neighbour or ghost.
 bool tile_count(Ctx& C, const SolverDev& S, std::vector<TileHdr>& hdr, int inst);
-// Places the lists of all headers (halo0, ext0) and allocates the table.
-void tile_place(Ctx& C, int nd, std::vector<TileHdr>& hdr, TileTab& t);
+// Places the lists of all headers (halo0, ext0) and allocates the table;
+// false if they exceed 32-bit offsets.
+bool tile_place(Ctx& C, int nd, std::vector<TileHdr>& hdr, TileTab& t);
 // Fills the lists of S's tiles, headers [tile0, tile0 + n); S's cells are
 // the cells tile0 * kTileCells onwards of the state arrays.
 void tile_fill(Ctx& C, const SolverDev& S, TileTab& t, long long tile0, long long n);

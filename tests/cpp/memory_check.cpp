@@ -162,8 +162,8 @@ static void short_of_memory() {
       try {
         DevBuf<char> y;
         y.alloc(200 * MB);
-      } catch (const Error&) {
-        failed = true;
+      } catch (const OutOfMemory& e) {
+        failed = e.code == HOM3G_ERR_HIP;
       }
       CHECK(failed && hipGetLastError() == hipSuccess, "no error, or one left for the next launch");
     }).join();
