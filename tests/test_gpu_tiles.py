@@ -1,8 +1,8 @@
 """First-order Euler stages on tiles (tile.hip) where their face lists have
-edges: fewer cells than a tile, exactly one tile and one more, remainders,
-grids of several levels whose interface tiles overflow the halo and
-extra-face places, boundary conditions with and without ghosts, periodic
-images, and a masked domain with cut boundaries; each against the oracle."""
+edges: fewer cells than a tile, exactly one tile, masked domains of one tile
+and one cell more, remainders, grids of several levels whose interface tiles
+overflow the halo and extra-face places, boundary conditions with and without
+ghosts, and periodic images; each against the oracle."""
 import numpy as np
 import pytest
 
@@ -31,9 +31,10 @@ def pair(nd, base, extra, radius, band, ti, bc, precision, kernel="tile"):
     og = O.Grid(nd, [0.0] * nd, [1.0] * nd).min_level(base)
     g = H.Grid(nd, [0.0] * nd, [1.0] * nd, base)
     if extra:
-        og.refine_region(base + extra, O.geom(O.GEOM_SPHERE, centre, [radius]), band)
+        for r in radius if isinstance(radius, tuple) else (radius,):
+            og.refine_region(base + extra, O.geom(O.GEOM_SPHERE, centre, [r]), band)
+            g.refine_region(base + extra, H.Sphere(centre, r), band)
         og.balance()
-        g.refine_region(base + extra, H.Sphere(centre, radius), band)
         g.balance()
     o = O.Solver(og, O.phys(physics=O.PHYS_EULER, nd=nd, ti=TI[ti], cfl=0.2))
     prm = fixed if bc == "dirichlet" else []
@@ -50,11 +51,117 @@ def pair(nd, base, extra, radius, band, ti, bc, precision, kernel="tile"):
     return o, s
 
 
+# thin rings of finer cells: tiles of the coarse cells between them
+RINGS = (2, 6, 1, tuple(0.02 + k * 3 / 64 for k in range(10)), 0.002)
 # (nd, base, extra, radius, band): 16 and 64 cells; one tile; ragged tiles of
-# refined grids; a ball refined twice (tiles over the level interfaces with
-# more than 384 halo cells and 128 extra faces a direction)
+# refined grids; a ball refined twice and rings, whose tiles over the level
+# interfaces have more halo cells and extra faces than places of their own
 GRIDS = [(2, 2, 0, 0, 0), (3, 2, 0, 0, 0), (2, 4, 0, 0, 0), (2, 4, 2, 0.2, 0.05), (3, 3, 1, 0.25, 0.1),
-         (3, 4, 2, 0.25, 0.02)]
+         (3, 4, 2, 0.25, 0.02), RINGS]
+PLACES = {2: (256, 256), 3: (384, 128)}  # halo cells and extra faces of a direction (tile.hpp)
+
+
+def list_lengths(s, nd):
+    """(halo cells, extra faces of each direction) of every tile of a solver
+    with zero-gradient boundaries."""
+    n, K = s.first_gc, 1 << (nd - 1)
+    nb, fine = s.topology()["neighbors"], s.fine_faces()
+    out = []
+    for base in range(0, n, 256):
+        end = min(n, base + 256)
+
+        def away(x):
+            return not base <= x < end
+        halo, ext = 0, [0] * nd
+        for c in range(base, end):
+            for d in range(nd):
+                lo, up = (c if v >= n else v for v in (int(nb[2 * d, c]), int(nb[2 * d + 1, c])))
+                if lo >= 0:
+                    halo += away(lo)
+                else:
+                    ext[d] += K
+                    halo += sum(away(x) for x in fine[-lo - 2])
+                if up < 0:
+                    ext[d] += K
+                    halo += sum(away(x) for x in fine[-up - 2])
+                elif away(up) or up == c or int(nb[2 * d, up]) != c:  # not the lower face of a cell of the tile
+                    ext[d] += 1
+                    halo += away(up)
+        out.append([halo] + ext)
+    return np.array(out)
+
+
+@pytest.mark.parametrize("grid", [(3, 4, 2, 0.25, 0.02), RINGS])
+def test_grids_overflow_the_places(grid):
+    """The grids above reach the lists past the places: halo cells read from
+    memory, and extra faces in more than one chunk in every direction."""
+    nd = grid[0]
+    _, s = pair(*grid, "ssp_rk3", "neumann", "fp64")
+    r = list_lengths(s, nd)
+    nhc, ce = PLACES[nd]
+    assert r[:, 0].max() > nhc
+    for d in range(nd):
+        assert r[:, 1 + d].max() > ce, d
+    # and tiles that do not
+    assert ((r[:, 0] <= nhc) & (r[:, 1:].max(1) <= ce)).any()
+
+
+def _box(nd, level, shape, mask, ti):
+    """A box of cells of a uniform grid, by its mask or its geometry: fixed
+    values at its upper x side, zero gradients elsewhere."""
+    import hom3_amd as H
+    h = 1.0 / (1 << level)
+    corner = [0.0] * nd if mask else [3 * h] * nd
+    size = [k * h for k in shape]
+    centre = [c + 0.5 * s for c, s in zip(corner, size)]
+    fixed = [0.1] * nd + [1.0, 2.5]
+    ic = [0.1] * nd + [1.0, 0.4 * (2.5 - 0.5 * nd * 0.01)]
+    og = O.Grid(nd, [0.0] * nd, [1.0] * nd).min_level(level)
+    g = H.Grid(nd, [0.0] * nd, [1.0] * nd, level)
+    o = O.Solver(og, O.phys(physics=O.PHYS_EULER, nd=nd, ti=TI[ti], cfl=0.2))
+    s = H.Solver(g, physics="euler", time_integration=ti, CFL=0.2, kernel="tile")
+    for d in range(nd):
+        for side in (0, 1):
+            x = list(centre)
+            x[d] = corner[d] + side * size[d]
+            normal = [0.0] * nd
+            normal[d] = -1.0 if side else 1.0
+            dirichlet = d == 0 and side == 1
+            o.append_bc(O.geom(O.GEOM_EDGE, x, normal), O.BC_EULER_DIRICHLET if dirichlet else O.BC_EULER_NEUMANN,
+                        fixed if dirichlet else [])
+            s.append_bc(H.Edge(x, normal), H.euler.bc.Dirichlet(fixed) if dirichlet else H.euler.bc.Neumann())
+    if mask:
+        # leaves in Morton order
+        m = np.arange(1 << (nd * level))
+        inside = np.ones(m.size, bool)
+        for d in range(nd):
+            inside &= sum(((m >> (nd * b + d)) & 1) << b for b in range(level)) < shape[d]
+        o.set_domain_mask(inside)
+        s.set_initial_domain(mask=inside)
+    else:
+        o.set_domain(O.geom(O.GEOM_SQUARE, centre, size, invert=True), +1)
+        s.set_initial_domain(H.invert(H.Square(centre, size)), +1)
+    for x in (o, s):
+        x.set_ic(O.IC_CONSTANT_PV, ic) if x is o else x.set_initial_condition(O.IC_CONSTANT_PV, ic)
+        x.set_perturbation(5, 0.02)
+        x.initialize()
+    return o, s
+
+
+@pytest.mark.parametrize("ti", list(TI))
+@pytest.mark.parametrize("nd,level,shape,mask", [(2, 9, (257, 1), True), (2, 5, (27, 19), False),
+                                                 (3, 4, (1, 1, 1), True), (3, 5, (19, 9, 3), False)])
+def test_masked_boxes_match_oracle(nd, level, shape, mask, ti):
+    """257, 513, 1 and 513 cells: whole tiles and one cell more, and a cell
+    that meets a ghost on every side."""
+    o, s = _box(nd, level, shape, mask, ti)
+    n = int(np.prod(shape))
+    assert s.first_gc == o.first_gc == n and n % 256 == 1
+    o.solve(6)
+    s.solve(6)
+    err = rel_l2(s.lhs, o.get("lhs"), nd)
+    assert np.max(err) <= 1e-12, err
+    assert abs(s.time() - o.time()) <= 1e-13 * o.time()
 
 
 @pytest.mark.parametrize("bc", ["neumann", "dirichlet", "periodic"])
@@ -113,6 +220,8 @@ def test_generic_forces_the_table_driven_kernel():
     H.append_bcs(m, H.Periodic())
     with pytest.raises(RuntimeError, match="tile kernel requested"):
         m.build()
+    with pytest.raises(RuntimeError, match="not built"):
+        m.solve(1)
 
 
 @pytest.mark.parametrize("nd,base", [(3, 4), (2, 6)])
