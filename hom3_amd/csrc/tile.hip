@@ -28,7 +28,7 @@
 // cells are read 1.3 times per cell on top of the compulsory bytes), 90% of
 // a device copy's rate.  FP64 holds three workgroups per CU (LDS and 168
 // VGPRs; at 174 it held two and the 0.82 M-leaf step took 0.18 ms), FP32 four
-// (115 VGPRs; held to 96 or 80 it spills and runs 13% and 60% slower).
+// (118-123 VGPRs; held to 96 or 80 it spills and runs 13% and 60% slower).
 //
 // 2D batches (which evaluated every face from both sides too), per step:
 // 512 instances of 76.7 M cells FP64 7.05 -> 5.12 ms, FP32 states 5.59 ->
@@ -599,7 +599,7 @@ void solver_build_tiles(Ctx& C, SolverDev& S) {
   try {
     if (!tile_count(C, S, hdr, 0) || !tile_place(C, S.nd, hdr, S.tile)) return;
   } catch (const OutOfMemory&) {
-    // the lists are 27 B per cell on top of the solver's tables and states,
+    // the lists are 21 (2D) or 25 B (3D) per cell on top of the solver's tables and states,
     // which are in place: it steps without them
     S.tile.release();
     return;
