@@ -189,6 +189,23 @@ def profile_vortex_run(H, level=12, steps=4):
     print(f"[bench] vortex profile run done (copy of 1 GiB in {ms:.3f} ms)", file=sys.stderr, flush=True)
 
 
+def profile_blast_run(H, steps=4):
+    """Short run for rocprofv3 on the refined blast: the shell (0.82 M leaves)
+    in FP64 and the ball (4.97 M) in FP32 state, on tiles and on the
+    table-driven kernel, then a 1 GiB device copy."""
+    from hom3_amd import cases
+    for kernel in ("auto", "generic"):
+        for band, prec in ((0.025, "fp64"), (0.2, "fp32")):
+            _, s, _ = cases.blast(H, base=6, extra=2, band=band, precision=prec, kernel=kernel)
+            s.solve(steps)
+            bad = s.check_state()
+            s.close()
+            if bad:
+                raise RuntimeError(f"blast {prec} {kernel}: {bad} non-physical cells")
+    ms = copy_calibration(H, 1 << 30)
+    print(f"[bench] blast profile run done (copy of 1 GiB in {ms:.3f} ms)", file=sys.stderr, flush=True)
+
+
 def copy_calibration(H, nbytes):
     import ctypes as C
     from hom3_amd import _lib
@@ -288,11 +305,12 @@ def bench_vortex_large(H, steps, level=12):
 
 
 def bench_blast(H, steps, band=0.025):
-    """3D Euler blast, base 64^3 + 2 levels where |r - 0.2| <= band, FP64
-    (table-driven kernel and the persistent kernel) and FP32 state (the
-    table-driven kernel with FP32 stage states, and the persistent kernel).  band 0.025 is the configured shell of width 0.05
-    (0.82 M leaves); band 0.2 refines the ball r <= 0.4, which gives the
-    configured 4-6 M leaves (4.97 M) and a state beyond the 256 MB MALL."""
+    """3D Euler blast, base 64^3 + 2 levels where |r - 0.2| <= band, FP64 and
+    FP32 state: the solver on tiles, a batch of one (the same stages, one
+    captured step per launch) and the table-driven kernel.  band 0.025 is the
+    configured shell of width 0.05 (0.82 M leaves); band 0.2 refines the ball
+    r <= 0.4, which gives the configured 4-6 M leaves (4.97 M) and a state
+    beyond the 256 MB MALL."""
     from hom3_amd import cases
     t0 = time.perf_counter()
     g, s, (nref, nbal) = cases.blast(H, base=6, extra=2, band=band)
@@ -305,20 +323,22 @@ def bench_blast(H, steps, band=0.025):
     B64 = H.Batch([s], "fp64")
     B32 = H.Batch([s], "fp32")
     sec = timed_solve(s, steps, 2)
-    out["fp64_table_driven"] = dict(mcs=round(n * 3 * steps / sec / 1e6, 1), ms_per_step=round(sec / steps * 1e3, 4))
-    _, s32, _ = cases.blast(H, base=6, extra=2, band=band, precision="fp32")
-    sec = timed_solve(s32, steps, 2)
-    l2, mx = state_error(s32.lhs[:, :n], s.lhs[:, :n], 3)
-    out["fp32_state_table_driven"] = dict(mcs=round(n * 3 * steps / sec / 1e6, 1),
-                                          ms_per_step=round(sec / steps * 1e3, 4),
-                                          vs_fp64_table_driven=dict(rel_l2=l2, rel_max=mx))
-    s32.close()
-    for tag, B in (("fp64_persistent", B64), ("fp32_state_persistent", B32)):
+    out["fp64_tiles"] = dict(mcs=round(n * 3 * steps / sec / 1e6, 1), ms_per_step=round(sec / steps * 1e3, 4))
+    q = s.lhs[:, :n]
+    for tag, kernel, prec in (("fp32_state_tiles", "auto", "fp32"), ("fp64_table_driven", "generic", "fp64"),
+                              ("fp32_state_table_driven", "generic", "fp32")):
+        _, x, _ = cases.blast(H, base=6, extra=2, band=band, precision=prec, kernel=kernel)
+        sec = timed_solve(x, steps, 2)
+        l2, mx = state_error(x.lhs[:, :n], q, 3)
+        out[tag] = dict(mcs=round(n * 3 * steps / sec / 1e6, 1), ms_per_step=round(sec / steps * 1e3, 4),
+                        vs_fp64_tiles=dict(rel_l2=l2, rel_max=mx))
+        x.close()
+    for tag, B in (("fp64_batch_of_one", B64), ("fp32_state_batch_of_one", B32)):
         cfg = B.autotune()
         B.solve(2)
         ms = B.time_solve(steps, graph=True)
         out[tag] = dict(mcs=round(n * 3 / (ms * 1e-3) / 1e6, 1), ms_per_step=round(ms, 4),
-                        config={k: cfg[k] for k in ("block", "tile", "grid")})
+                        config=dict(grid=cfg["grid"], tiles=B.config()["items"]))
     q64, q32 = B64.state(0), B32.state(0)
     l2, mx = state_error(q32, q64, 3)
     out["fp32_vs_fp64"] = dict(vars=["rho_u0", "rho_u1", "rho_u2", "rho", "rho_E"], rel_l2=l2, rel_max=mx)
@@ -331,7 +351,7 @@ def bench_blast(H, steps, band=0.025):
 def bench_batch(H, n_inst, steps, seed=2024):
     """512 independent 2D four-quadrant instances, sides 64..512 (level
     uniform over 6..9), 0-2 refinement levels inside a seeded disc, one
-    persistent kernel per stage, hipGraph steps, autotuned launch shape."""
+    sweep over all tiles per stage, hipGraph steps, autotuned number of workgroups."""
     from hom3_amd.batch import build_instance
     t0 = time.perf_counter()
     prms = H.four_quadrant_instances(seed, n_inst)
@@ -352,9 +372,10 @@ def bench_batch(H, n_inst, steps, seed=2024):
         B.solve(2)
         ms_g = B.time_solve(steps, graph=True)
         ms_s = B.time_solve(10, graph=False)
-        bytes_cs = ((8.0 / 3.0) * 4 * 8 if tag == "fp64" else 16.0 * 4) + 4 * 4
+        # the states and the tile lists (faces 8, level 1, halo cells 4, extra faces 8)
+        bytes_cs = ((8.0 / 3.0) * 4 * 8 if tag == "fp64" else 16.0 * 4) + 21
         out[tag] = dict(mcs=round(ncell * 3 / (ms_g * 1e-3) / 1e6, 1), ms_per_step_graph=round(ms_g, 4),
-                        ms_per_step_stream=round(ms_s, 4), config={k: cfg[k] for k in ("block", "tile", "grid")},
+                        ms_per_step_stream=round(ms_s, 4), config=dict(grid=cfg["grid"], tiles=B.config()["items"]),
                         autotune_stage_ms=round(cfg["stage_ms"], 4),
                         achieved_gbs=round(bytes_cs * ncell * 3 / (ms_g * 1e-3) / 1e9, 1))
     # both batches have taken the same steps: FP32 state against FP64, worst
@@ -524,7 +545,9 @@ def write_traffic(fetch_csv, write_csv, level=8, out_path=TRAFFIC_JSON):
             acc.setdefault((name, disp), 0.0)
             acc[(name, disp)] += val
         return acc
-    stage_key = "k_brick<3, 1, false, double, double, double, false>"
+    # full bricks (the argument after the types); on 256^3 the dt has a launch
+    # of its own, so the three stages are one kernel
+    stage_key = "k_brick<3, 1, false, double, double, double, false"
     out = {}
     for counter, path in (("FETCH_SIZE", fetch_csv), ("WRITE_SIZE", write_csv)):
         acc = per_kernel(path, counter)
@@ -597,6 +620,9 @@ def main():
     ap.add_argument("--copy-sweep", action="store_true", help="only the device-copy bandwidth sweep")
     ap.add_argument("--write-traffic", nargs=2, metavar=("FETCH_CSV", "WRITE_CSV"),
                     help="write profiles/tgv256_fp64_stage_traffic.json from two rocprofv3 --pmc runs")
+    ap.add_argument("--profile-blast", action="store_true",
+                    help="profiling run of the refined blast: 4 steps of the shell and the ball on tiles and on the "
+                         "table-driven kernel + a 1 GiB copy")
     ap.add_argument("--profile-batch", action="store_true",
                     help="profiling run of the 512-instance batch: 3 FP64 + 3 FP32-state steps + a 1 GiB copy")
     args = ap.parse_args()
@@ -617,6 +643,9 @@ def main():
         return
     if args.profile_vortex:
         profile_vortex_run(H)
+        return
+    if args.profile_blast:
+        profile_blast_run(H)
         return
     if args.profile_batch:
         profile_batch_run(H, args.batch_n)

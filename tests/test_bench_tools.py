@@ -4,6 +4,8 @@ run), with the provenance of the kernel sources it was measured on."""
 import csv
 import json
 
+import pytest
+
 import bench
 
 
@@ -16,8 +18,11 @@ def _write_pmc(path, counter, rows):
             w.writerow(dict(Dispatch_Id=disp, Kernel_Name=name, Counter_Name=counter, Counter_Value=val))
 
 
-def test_write_traffic_scales_by_the_copy(tmp_path):
-    stage = "void hom3g::(anonymous namespace)::k_brick<3, 1, false, double, double, double, false>(args)"
+# the stage kernel by its name, alone and with the template arguments that follow
+@pytest.mark.parametrize("tail", ["false", "false, false"])
+def test_write_traffic_scales_by_the_copy(tmp_path, tail):
+    stage = f"void hom3g::(anonymous namespace)::k_brick<3, 1, false, double, double, double, {tail}>(args)"
+    tiled = "void hom3g::(anonymous namespace)::k_brick<3, 1, false, double, double, double, true, false>(args)"
     copy = "hom3g::(anonymous namespace)::k_copy(double4 const*, double4*, long long)"
     gib_kib = float(1 << 30) / 1024
     # FETCH counts half of a streaming read (factor 2), WRITE all of it
@@ -25,6 +30,9 @@ def test_write_traffic_scales_by_the_copy(tmp_path):
     write = [(i, stage, 500.0) for i in range(8)] + [(100, copy, gib_kib)]
     # a second counter row of the same dispatch (another XCD) adds up
     fetch.append((0, stage, 0.0))
+    # tiled bricks are another kernel
+    fetch.append((50, tiled, 1e9))
+    write.append((50, tiled, 1e9))
     fa, wa = tmp_path / "f.csv", tmp_path / "w.csv"
     _write_pmc(fa, "FETCH_SIZE", fetch)
     _write_pmc(wa, "WRITE_SIZE", write)
