@@ -350,7 +350,8 @@ __device__ __forceinline__ void brick_direction(Smem<ND, PHYS, MUSCL, TC>& s, co
 template <int ND, int PHYS, bool MUSCL, class TC>
 __device__ __forceinline__ void put_prims(Smem<ND, PHYS, MUSCL, TC>& s, int i, const TC* q, const PhysConst& pc) {
   TC p, ia;
-  brick_prims<ND, TC>(q, TC(pc.gamma), TC(pc.gm1), p, ia);
+  if constexpr (PHYS == HOM3G_EULER) euler_prims<ND, TC>(q, TC(pc.gamma), TC(pc.gm1), p, ia);
+  else brick_prims<ND, TC>(q, TC(pc.gamma), TC(pc.gm1), p, ia);
   s.p[i] = p;
   s.iar[i] = ia;
 }

@@ -97,6 +97,24 @@ __device__ __forceinline__ void brick_prims(const T* q, T gamma, T gm1, T& p, T&
   ia = fast_rsq(gamma * p * q[ND]);
 }
 
+// The same for Euler states, which come in any units: in FP32 the products
+// p rho and |rho u|^2 leave its range where p and rho themselves are far from
+// doing so (a gas of 1e-24), so those are formed from p / rho and u.  (The CNS
+// states are scaled by the stagnation values.)
+template <int ND, class T>
+__device__ __forceinline__ void euler_prims(const T* q, T gamma, T gm1, T& p, T& ia) {
+  if constexpr (sizeof(T) == 4) {
+    const T ir = dev_rcp(q[ND]);
+    T m = T(0);
+#pragma unroll
+    for (int d = 0; d < ND; ++d) m += q[d] * (q[d] * ir);
+    p = gm1 * (q[ND + 1] - T(0.5) * m);
+    ia = fast_rsq(gamma * (p * ir)) * ir;
+  } else {
+    brick_prims<ND, T>(q, gamma, gm1, p, ia);
+  }
+}
+
 // Cell primitives: u_d = rho u_d / rho, p = (g-1)(rho E - 0.5 rho |u|^2), a = sqrt(g p / rho)
 template <int ND, class T>
 struct Prim {

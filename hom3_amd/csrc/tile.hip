@@ -289,7 +289,7 @@ __device__ __forceinline__ void fetch(const TileSmem<ND, TC>& s, const TileArgs&
                                       int pos, CellState<ND, TC>& w) {
   if (__builtin_expect(pos >= T + TileCfg<ND>::NHC, 0)) {
     load_state<ND, TC, TIn>(A, A.t.halo_more[halo0 + pos - T - TileCfg<ND>::NHC], w.q);
-    brick_prims<ND, TC>(w.q, TC(pc.gamma), TC(pc.gm1), w.p, w.iar);
+    euler_prims<ND, TC>(w.q, TC(pc.gamma), TC(pc.gm1), w.p, w.iar);
     return;
   }
 #pragma unroll
@@ -426,14 +426,14 @@ __global__ void __launch_bounds__(T, ND == 3 && sizeof(TC) == 8 ? 3 : 4) k_tile_
       if (j < NHC && j < H.nh) {
         CellState<ND, TC> w;
         load_state<ND, TC, TIn>(A, hid[r], w.q);
-        brick_prims<ND, TC>(w.q, TC(pc.gamma), TC(pc.gm1), w.p, w.iar);
+        euler_prims<ND, TC>(w.q, TC(pc.gamma), TC(pc.gm1), w.p, w.iar);
 #pragma unroll
         for (int v = 0; v < NV; ++v) s.q[v][T + j] = w.q[v];
         s.p[T + j] = w.p;
         s.iar[T + j] = w.iar;
       }
     }
-    brick_prims<ND, TC>(own.q, TC(pc.gamma), TC(pc.gm1), own.p, own.iar);
+    euler_prims<ND, TC>(own.q, TC(pc.gamma), TC(pc.gm1), own.p, own.iar);
 #pragma unroll
     for (int v = 0; v < NV; ++v) s.q[v][i] = own.q[v];
     s.p[i] = own.p;

@@ -268,3 +268,36 @@ def test_fused_dt_equals_the_reduction():
     _, a = pair(2, 4, 2, 0.2, 0.05, "ssp_rk3", "neumann", "fp64")
     a.solve(6)
     np.testing.assert_array_equal(a.lhs, s.lhs)
+
+
+@pytest.mark.parametrize("kernel", ["tile", "generic", "auto"])
+def test_fp32_state_does_not_depend_on_the_units(kernel):
+    """The Euler equations do not change when density and pressure are scaled
+    together, and a power of two changes no rounding: FP32 stage states at
+    2^-80 (a gas of 1e-24) take the same steps as at 1.  kernel auto: the
+    bricks of a uniform grid."""
+    import hom3_amd as H
+    args = (3, 4, 0, 0, 0) if kernel == "auto" else (3, 3, 1, 0.25, 0.1)
+    _, s = pair(*args, "ssp_rk3", "neumann", "fp32", kernel=kernel)
+    assert s.kernel() == ("brick" if kernel == "auto" else "generic")
+    q0, n = s.lhs.copy(), s.first_gc
+    out = []
+    for scale in (1.0, 2.0 ** -80):
+        s.set_lhs(q0 * scale)
+        s.reset_time(0.0, 0.0, 0)
+        s.solve(5)
+        out.append((s.lhs[:, :n] / scale, s.time()))
+    # (what underflows is 2^-46 of a term that it is added to)
+    assert np.max(rel_l2(out[1][0], out[0][0], 3)) <= 1e-7
+    assert abs(out[1][1] - out[0][1]) <= 1e-7 * out[0][1]
+    if kernel != "tile":
+        return
+    b = []
+    for scale in (1.0, 2.0 ** -80):
+        s.set_lhs(q0 * scale)
+        s.reset_time(0.0, 0.0, 0)
+        B = H.Batch([s], "fp32")
+        B.solve(5)
+        b.append(B.state(0) / scale)
+        B.close()
+    assert np.max(rel_l2(b[1], b[0], 3)) <= 1e-7
