@@ -20,20 +20,21 @@
 // direction), in chunks of CE.
 //
 // Measured (one MI355X, refined blast, per step of three stages): 0.82 M
-// leaves FP64 0.258 -> 0.156 ms, 4.97 M leaves FP32 states 0.70 -> 0.45 ms
+// leaves FP64 0.24 -> 0.148 ms, 4.97 M leaves FP32 states 0.67 -> 0.455 ms
 // against the table-driven kernel and its separate ghost fills, CFL
-// reduction and advance.  A tile takes 7-9 us, most of it waiting: the chain
-// from the halo list to the halo states to the first face, and the two
-// barriers per direction; at 5 M leaves the stages move 4.6 TB/s (the halo
-// cells are read 1.3 times per cell on top of the compulsory bytes), 90% of
-// a device copy's rate.  FP64 holds three workgroups per CU (LDS and 168
+// reduction and advance; per cell-stage 490-600 VALU instead of 1,000 (FP64).
+// A tile takes 7-9 us, 60% of it waiting: the chain from the halo list to the
+// halo states to the first face, and the two barriers per direction; at 5 M
+// leaves the stages read and write 5.2-5.6 TB/s (the halo cells are read 1.3
+// times per cell on top of the compulsory bytes, in part from the caches), a
+// device copy 4.9.  FP64 holds three workgroups per CU (LDS and 168
 // VGPRs; at 174 it held two and the 0.82 M-leaf step took 0.18 ms), FP32 four
 // (118-123 VGPRs; held to 96 or 80 it spills and runs 13% and 60% slower).
 //
 // 2D batches (which evaluated every face from both sides too), per step:
-// 512 instances of 76.7 M cells FP64 7.05 -> 5.12 ms, FP32 states 5.59 ->
-// 4.14 ms; a pass of 40 steps of 12 instances (base grids 64^2 to 256^2, FP64)
-// 4.54 -> 3.78 ms.
+// 512 instances of 76.7 M cells FP64 7.05 -> 6.26 ms, FP32 states 5.59 ->
+// 4.41 ms; a pass of 40 steps of 12 instances (base grids 64^2 to 256^2, FP64)
+// 4.47 -> 3.42 ms.
 //
 // Boundaries.  A zero-gradient Neumann ghost holds a copy of its boundary
 // cell and a periodic one a copy of its image, so their faces read that cell
