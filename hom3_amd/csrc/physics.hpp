@@ -168,8 +168,8 @@ __device__ __forceinline__ void ausm_flux(const T* qL, const Prim<ND, T>& wL, co
   f[D] += p_i;
 }
 
-// First-order and MUSCL Euler paths (table-driven, batched and brick
-// kernels): the primitives with one refined reciprocal of rho instead of
+// First-order and MUSCL Euler paths (table-driven and MUSCL brick kernels):
+// the primitives with one refined reciprocal of rho instead of
 // nd + 1 divisions, and AUSM with the Mach numbers from refined reciprocals
 // of a and the supersonic pressure weights in closed form (exactly 1 or 0).
 // Values agree with primitives() / ausm_flux() to rounding.

@@ -25,15 +25,15 @@
 // reduction and advance; per cell-stage 490-600 VALU instead of 1,000 (FP64).
 // A tile takes 7-9 us, 60% of it waiting: the chain from the halo list to the
 // halo states to the first face, and the two barriers per direction; at 5 M
-// leaves the stages read and write 5.2-5.6 TB/s (the halo cells are read 1.3
+// leaves the stages read and write 5.2-5.5 TB/s (the halo cells are read 1.3
 // times per cell on top of the compulsory bytes, in part from the caches), a
 // device copy 4.9.  FP64 holds three workgroups per CU (LDS and 168
 // VGPRs; at 174 it held two and the 0.82 M-leaf step took 0.18 ms), FP32 four
 // (118-123 VGPRs; held to 96 or 80 it spills and runs 13% and 60% slower).
 //
 // 2D batches (which evaluated every face from both sides too), per step:
-// 512 instances of 76.7 M cells FP64 7.05 -> 6.26 ms, FP32 states 5.59 ->
-// 4.41 ms; a pass of 40 steps of 12 instances (base grids 64^2 to 256^2, FP64)
+// 512 instances of 76.7 M cells FP64 7.05 -> 6.25 ms, FP32 states 5.59 ->
+// 4.32 ms; a pass of 40 steps of 12 instances (base grids 64^2 to 256^2, FP64)
 // 4.47 -> 3.42 ms.
 //
 // Boundaries.  A zero-gradient Neumann ghost holds a copy of its boundary

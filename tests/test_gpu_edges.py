@@ -45,7 +45,7 @@ def test_brick_kernel_on_a_refined_grid_is_an_error():
     with pytest.raises(Hom3gError) as e:
         s.initialize()
     assert e.value.code == ERR_ARG and "brick" in str(e.value)
-    _, s2 = _blast(H, 3, refine=True)  # auto: the table-driven kernel
+    _, s2 = _blast(H, 3, refine=True)  # auto: no bricks
     s2.initialize()
     assert s2.kernel() == "generic"
 

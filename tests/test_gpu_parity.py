@@ -243,8 +243,8 @@ def _heat(nd, level, neumann=False):
 
 
 # every scenario with the kernel picked at build ("auto": bricks, tiled
-# bricks where the cells fall into whole bricks, else table-driven) and with
-# the table-driven kernel forced
+# bricks where the cells fall into whole bricks, else tiles for first-order
+# Euler, else table-driven) and with the table-driven kernel forced
 _PARITY_CASES = [(n, "auto") for n in STEP_SCENARIOS if not n.endswith("generic")] + \
     [(n, "generic") for n in STEP_SCENARIOS if not n.startswith("heat")]
 

@@ -20,7 +20,7 @@ CASES = {
 TI = {"euler_forward": O.TI_EULER_FWD, "ssp_rk3": O.TI_SSP_RK3}
 
 
-def build_pair(name, seed=7, amp=0.01, precision="fp64"):
+def build_pair(name, seed=7, amp=0.01, precision="fp64", kernel="auto"):
     import hom3_amd as H
     nd, base, extra, centre, radius, band, ic, nsteps, ti, cfl = CASES[name]
     xmin, xmax = [0.0] * nd, [1.0] * nd
@@ -36,7 +36,7 @@ def build_pair(name, seed=7, amp=0.01, precision="fp64"):
     g = H.Grid(nd, xmin, xmax, base)
     nref = g.refine_region(base + extra, H.Sphere(centre, radius), band)
     nbal = g.balance()
-    s = H.Solver(g, physics="euler", time_integration=ti, CFL=cfl, precision=precision)
+    s = H.Solver(g, physics="euler", time_integration=ti, CFL=cfl, precision=precision, kernel=kernel)
     H.append_bcs(s, H.euler.bc.Neumann())
     s.set_initial_condition(*ic)
     s.set_perturbation(seed, amp)
@@ -63,9 +63,11 @@ def test_refined_topology_bit_exact(name):
     assert s.kernel() == "generic"
 
 
+# auto: the tiles; generic: the table-driven kernel
+@pytest.mark.parametrize("kernel", ["auto", "generic"])
 @pytest.mark.parametrize("name", list(CASES))
-def test_refined_steps_match_oracle(name):
-    (og, o), (g, s), nsteps, _ = build_pair(name)
+def test_refined_steps_match_oracle(name, kernel):
+    (og, o), (g, s), nsteps, _ = build_pair(name, kernel=kernel)
     nd = o.nd
     n = o.first_gc
     # initial condition + perturbation
@@ -80,14 +82,15 @@ def test_refined_steps_match_oracle(name):
     np.testing.assert_allclose(s.conservation_sums(), o.conservation_sums(), rtol=1e-12, atol=1e-15)
 
 
+@pytest.mark.parametrize("kernel", ["auto", "generic"])
 @pytest.mark.parametrize("name", list(CASES))
-def test_refined_fp32_state_against_oracle(name):
-    """FP32 stage states on the table-driven kernel of a refined grid (the
-    stage buffers and the fluxes in FP32, the RK combination and U^n in
-    FP64):
+def test_refined_fp32_state_against_oracle(name, kernel):
+    """FP32 stage states on a refined grid, on tiles and on the table-driven
+    kernel (the stage buffers and the fluxes in FP32, the RK combination and
+    U^n in FP64):
     relative L2 <= 1e-5 per variable against the FP64 oracle after the
     case's steps (forward Euler has no stage buffers: the FP64 result)."""
-    (og, o), (g, s), nsteps, _ = build_pair(name, precision="fp32")
+    (og, o), (g, s), nsteps, _ = build_pair(name, precision="fp32", kernel=kernel)
     assert s.kernel() == "generic"
     nd = o.nd
     n = o.first_gc

@@ -57,12 +57,13 @@ def test_brick_tgv_fp32_replays_match_eager():
     _check_replays(a, b)
 
 
-def test_generic_blast_replays_match_eager():
+@pytest.mark.parametrize("kernel", ["tile", "generic"])
+def test_generic_blast_replays_match_eager(kernel):
     import hom3_amd as H
     from hom3_amd import cases
 
     def make():
-        g, s, _ = cases.blast(H, base=4, extra=1)
+        g, s, _ = cases.blast(H, base=4, extra=1, kernel=kernel)
         return g, s
     (_, a), (_, b) = _pair(make)
     assert b.kernel() == "generic"
